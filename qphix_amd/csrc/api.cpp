@@ -171,8 +171,6 @@ extern "C" int qphix_init(int device) {
   HIPCHK(hipHostMalloc(&g_hres, sizeof(double) * kResults, hipHostMallocDefault));
   HIPCHK(hipEventCreate(&g_ev0));
   HIPCHK(hipEventCreate(&g_ev1));
-  // the device address of the allocation-free clover build's static scratch
-  HIPCHK(fld_noalloc_init(device));
   g_init = true;
   return QPHIX_OK;
 }
@@ -434,12 +432,8 @@ extern "C" int qphix_clover_build(const qphix_geom *g, const void *u0, const voi
   HIPCHK(hipStreamSynchronize(g_stream));
   return QPHIX_OK;
 }
-// The same build with no allocation, free or synchronisation: the FP64
-// scratch is a static device array of a fixed size (kNoAllocSites sites),
-// looked up by qphix_init, which must have run (it is the call that
-// allocates). Lattices of any size are built in chunks of that many sites.
-// Stream-ordered on the library stream; two calls that overlap on one device
-// share the scratch and race.
+// The same build without the closing synchronisation, for callers that may not
+// allocate either: qphix_init (the call that allocates) must have run.
 extern "C" int qphix_clover_build_noalloc(const qphix_geom *g, const void *u0, const void *u1, double csw_r,
                                           double csw_t, double diag_mass, int cb, int what, double mu, double eps,
                                           void *out) {
@@ -447,8 +441,7 @@ extern "C" int qphix_clover_build_noalloc(const qphix_geom *g, const void *u0, c
   CHKPTR(g); CHKPTR(u0); CHKPTR(u1); CHKPTR(out);
   TRY(check_cb(cb));
   if (what < QPHIX_CLOV_A || what > QPHIX_CLOV_ND_OFF) return fail(QPHIX_EDOMAIN, "unknown clover output %d", what);
-  HIPCHK(fld_clover_build_noalloc(g->d, u0, u1, 0.5 * csw_r, 0.5 * csw_t, diag_mass, cb, what, mu, eps, out,
-                                  g_device, g_stream));
+  HIPCHK(fld_clover_build(g->d, u0, u1, 0.5 * csw_r, 0.5 * csw_t, diag_mass, cb, what, mu, eps, out, g_stream));
   return QPHIX_OK;
 }
 

@@ -270,127 +270,153 @@ __global__ void k_convert_words(void *out, const void *in, size_t vs, long vh) {
 typedef cx<double> zd;
 
 // ---------------------------------------------------------------------------
-// clover term: field strength per plane, then per chiral block the Hermitian
-// 6x6 matrix and what is asked of it, then the store in the field precision.
-// Three launches over chunks of sites keep every work-item's arrays in
-// registers (no private memory); the FP64 intermediates live in a chunk-sized
-// scratch allocated by the host launcher.
+// clover term: one kernel from the links to the stored blocks.
+//
+// A work-group of two wavefronts takes 64 sites: each wavefront computes three
+// of the six planes of the field strength of its lane's site and leaves their
+// nine reals (F is anti-Hermitian) in LDS; after a barrier wavefront b builds
+// chiral block b from them, inverts it where asked and stores it in the field
+// precision. Nothing but the links is read and nothing but the result is
+// written. Bound: the 96 link reads a site (12 distinct ones a plane), most of
+// them from beyond the L2, whose 4 MB cannot hold the t neighbours of the
+// 8192 sites an XCD has in flight; the FP64 products are a third of the time
+// (as FMA chains, a third fewer instructions, they gave 1%, not kept). The
+// work-groups of an XCD walk one contiguous range (551 us without that).
+// Measured at 24^3x48, FP64, A^-1: 467 us a build; the form before, eight
+// kernels per 2^20 sites through 252 doubles of scratch a site, took 772 us
+// of kernels and 19 ms with the scratch allocated and freed by each build.
 // ---------------------------------------------------------------------------
 
-// U_mu at site c (either checkerboard): link 2mu+1 of the array of c's own
-// checkerboard, reading only the words that hold it
-template <int P, bool C12, int MU>
-__device__ inline void site_link(const void *const u[2], size_t vs, const Lat &l, const int c[4], zd (&U)[3][3]) {
+// U_mu at a site: link 2 mu + 1 of its record. The link's place within its
+// first word is the same for every mu (2 mu + 1 is odd), so mu may be a
+// run-time value. load() reads the words that hold it, make() rebuilds it.
+template <int P, bool C12> struct SiteLink {
   typedef GaugeLayout<P, C12> GL;
   typedef typename PT<P>::calc T;
-  constexpr int pw = PT<P>::per_word;
-  constexpr int first = (2 * MU + 1) * GL::link_reals;
-  constexpr int w0 = first / pw;
-  constexpr int w1 = (first + GL::link_reals + pw - 1) / pw;
-  T buf[(w1 - w0) * pw];
-  load_range<P, GL::nw, w0, w1 - w0>(u[cb_of(c)], vs, cb_site(l, c), buf);
-  cx<T> Ut[3][3];
-  make_link<C12>(buf + (first - w0 * pw), Ut);
+  static constexpr int pw = PT<P>::per_word;
+  static constexpr int off = GL::link_reals % pw;
+  static constexpr int w0 = GL::link_reals / pw;
+  static constexpr int nwl = (off + GL::link_reals + pw - 1) / pw;
+  T buf[nwl * pw];
+  __device__ inline void load(const void *u, size_t vs, int mu, unsigned s) {
 #pragma unroll
-  for (int a = 0; a < 3; a++)
+    for (int w = 0; w < nwl; w++)
+      Word<P>::template load<false>(u, widx(s, w0 + mu * GL::pair_words + w, GL::nw), buf + w * pw);
+    if constexpr (PT<P>::scaled) {
+      const T sc = site_scale<P>(u, vs, s, GL::nw);
 #pragma unroll
-    for (int b = 0; b < 3; b++) U[a][b] = mk((double)Ut[a][b].r, (double)Ut[a][b].i);
-}
-
-// X = U (FIRST) or X = X U, with U = U_mu(c) or its adjoint (DAG)
-template <int P, bool C12, int MU, bool DAG, bool FIRST>
-__device__ inline void leaf_mul(const void *const u[2], size_t vs, const Lat &l, const int c[4], zd (&X)[3][3]) {
-  zd U[3][3];
-  site_link<P, C12, MU>(u, vs, l, c, U);
-  if constexpr (FIRST) {
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++) X[a][b] = DAG ? conj(U[b][a]) : U[a][b];
-  } else {
-    zd Y[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++) {
-        zd t = mk(0.0, 0.0);
-#pragma unroll
-        for (int k = 0; k < 3; k++) t = t + X[a][k] * (DAG ? conj(U[b][k]) : U[k][b]);
-        Y[a][b] = t;
-      }
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++) X[a][b] = Y[a][b];
+      for (int k = 0; k < nwl * pw; k++) buf[k] *= sc;
+    }
   }
+  __device__ inline void make(zd (&U)[3][3]) const {
+    cx<T> Ut[3][3];
+    make_link<C12>(buf + off, Ut);
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int b = 0; b < 3; b++) U[a][b] = mk((double)Ut[a][b].r, (double)Ut[a][b].i);
+  }
+};
+
+// a site of the full lattice: coordinates, checkerboard site and checkerboard
+struct CloverSite {
+  int c0, c1, c2, c3;
+};
+__device__ inline int wrapped(int c, int d, int n) {
+  c += d;
+  return c < 0 ? c + n : c >= n ? c - n : c;
+}
+__device__ inline void shift(CloverSite &x, const Lat &l, int mu, int d) {
+  if (mu == 0) x.c0 = wrapped(x.c0, d, l.L[0]);
+  else if (mu == 1) x.c1 = wrapped(x.c1, d, l.L[1]);
+  else if (mu == 2) x.c2 = wrapped(x.c2, d, l.L[2]);
+  else x.c3 = wrapped(x.c3, d, l.L[3]);
 }
 
-__device__ inline void shifted(const Lat &l, const int c[4], int mu, int dm, int nu, int dn, int o[4]) {
-#pragma unroll
-  for (int k = 0; k < 4; k++) o[k] = c[k];
-  o[mu] = (o[mu] + dm + l.L[mu]) % l.L[mu];
-  o[nu] = (o[nu] + dn + l.L[nu]) % l.L[nu];
-}
-
-// coef * F_{MU NU}(x) = coef * (Q - Q^+) / 8, Q the sum of the four clover
-// leaves at x (tests/mesfield.cc:24-64), for the chunk sites s0 + j; written
-// as 18 doubles, element e at F[e * n + j]
-template <int P, bool C12, int MU, int NU>
-__global__ void __launch_bounds__(128) k_field_strength(const void *u0, const void *u1, size_t vs, Lat l, int cb,
-                                                        long s0, long n, double coef, double *F) {
-  const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const void *const u[2] = {u0, u1};
-  int x[4], xpm[4], xpn[4], xmm[4], xmmpn[4], xmmmn[4], xmn[4], xpmmn[4];
-  cb_coords(l, cb, s0 + j, x);
-  shifted(l, x, MU, 1, NU, 0, xpm);     // x + mu
-  shifted(l, x, MU, 0, NU, 1, xpn);     // x + nu
-  shifted(l, x, MU, -1, NU, 0, xmm);    // x - mu
-  shifted(l, x, MU, -1, NU, 1, xmmpn);  // x - mu + nu
-  shifted(l, x, MU, -1, NU, -1, xmmmn); // x - mu - nu
-  shifted(l, x, MU, 0, NU, -1, xmn);    // x - nu
-  shifted(l, x, MU, 1, NU, -1, xpmmn);  // x + mu - nu
-  zd Q[3][3], X[3][3];
-  // U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
-  leaf_mul<P, C12, MU, false, true>(u, vs, l, x, X);
-  leaf_mul<P, C12, NU, false, false>(u, vs, l, xpm, X);
-  leaf_mul<P, C12, MU, true, false>(u, vs, l, xpn, X);
-  leaf_mul<P, C12, NU, true, false>(u, vs, l, x, X);
-#pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int b = 0; b < 3; b++) Q[a][b] = X[a][b];
-  // U_nu(x) U_mu(x-mu+nu)^+ U_nu(x-mu)^+ U_mu(x-mu)
-  leaf_mul<P, C12, NU, false, true>(u, vs, l, x, X);
-  leaf_mul<P, C12, MU, true, false>(u, vs, l, xmmpn, X);
-  leaf_mul<P, C12, NU, true, false>(u, vs, l, xmm, X);
-  leaf_mul<P, C12, MU, false, false>(u, vs, l, xmm, X);
-#pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int b = 0; b < 3; b++) Q[a][b] = Q[a][b] + X[a][b];
-  // U_mu(x-mu)^+ U_nu(x-mu-nu)^+ U_mu(x-mu-nu) U_nu(x-nu)
-  leaf_mul<P, C12, MU, true, true>(u, vs, l, xmm, X);
-  leaf_mul<P, C12, NU, true, false>(u, vs, l, xmmmn, X);
-  leaf_mul<P, C12, MU, false, false>(u, vs, l, xmmmn, X);
-  leaf_mul<P, C12, NU, false, false>(u, vs, l, xmn, X);
-#pragma unroll
-  for (int a = 0; a < 3; a++)
-#pragma unroll
-    for (int b = 0; b < 3; b++) Q[a][b] = Q[a][b] + X[a][b];
-  // U_nu(x-nu)^+ U_mu(x-nu) U_nu(x-nu+mu) U_mu(x)^+
-  leaf_mul<P, C12, NU, true, true>(u, vs, l, xmn, X);
-  leaf_mul<P, C12, MU, false, false>(u, vs, l, xmn, X);
-  leaf_mul<P, C12, NU, false, false>(u, vs, l, xpmmn, X);
-  leaf_mul<P, C12, MU, true, false>(u, vs, l, x, X);
-  const double f = 0.125 * coef;
+// X = X U, or X U^+ (DAG)
+template <bool DAG> __device__ inline void times_link(zd (&X)[3][3], const zd (&U)[3][3]) {
+  zd Y[3][3];
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
     for (int b = 0; b < 3; b++) {
-      const zd v = scale(f, (Q[a][b] + X[a][b]) - conj(Q[b][a] + X[b][a]));
-      F[(2 * (3 * a + b)) * n + j] = v.r;
-      F[(2 * (3 * a + b) + 1) * n + j] = v.i;
+      zd t = mk(0.0, 0.0);
+#pragma unroll
+      for (int k = 0; k < 3; k++) t = t + X[a][k] * (DAG ? conj(U[b][k]) : U[k][b]);
+      Y[a][b] = t;
+    }
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) X[a][b] = Y[a][b];
+}
+
+constexpr int kCloverSites = 64;  // sites per work-group
+constexpr int kPlaneReals = 9;    // reals of an anti-Hermitian 3x3 matrix
+
+// coef * F_{mu nu}(x) = coef * (Q - Q^+) / 8, Q the sum of the four clover
+// leaves at x (tests/mesfield.cc:24-64); its diagonal (imaginary) in
+// F[0..2], (1,0), (2,0), (2,1) in F[3..8], entry e of lane j at F[e * 64 + j].
+// Leaf q walks the plaquette's four steps +mu +nu -mu -nu from step q on, so
+// the sixteen factors are one loop: unrolled, the compiler kept the twelve
+// distinct links live (512 registers and a spill); rolled, with the next
+// link's load ahead of the product, it fits two wavefronts per SIMD.
+template <int P, bool C12>
+__device__ inline void field_strength(const void *u0, const void *u1, size_t vs, const Lat &l, const CloverSite &x,
+                                      int mu, int nu, double coef, double *F) {
+  zd Q[3][3], X[3][3];
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) Q[a][b] = X[a][b] = mk(0.0, 0.0);
+  CloverSite pos = x;
+  SiteLink<P, C12> link;
+  // the link of factor n (a step against its direction takes the link of the
+  // site it leads to), and the step
+  auto fetch = [&](int n) {
+    if ((n & 3) == 0) pos = x;
+    const int k = ((n >> 2) + n) & 3, dir = (k & 1) ? nu : mu;
+    if (k >> 1) shift(pos, l, dir, -1);
+    const unsigned s = (((unsigned)pos.c3 * l.L[2] + pos.c2) * l.L[1] + pos.c1) * l.nxh + ((unsigned)pos.c0 >> 1);
+    link.load(((pos.c0 + pos.c1 + pos.c2 + pos.c3) & 1) ? u1 : u0, vs, dir, s);
+    if (!(k >> 1)) shift(pos, l, dir, 1);
+  };
+  fetch(0);
+#pragma nounroll
+  for (int n = 0; n < 16; n++) {
+    zd U[3][3];
+    link.make(U);
+    if (n < 15) fetch(n + 1);
+    const bool dag = (((n >> 2) + n) & 2) != 0;
+    if ((n & 3) == 0) {
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) X[a][b] = dag ? conj(U[b][a]) : U[a][b];
+    } else if (dag) {
+      times_link<true>(X, U);
+    } else {
+      times_link<false>(X, U);
+    }
+    if ((n & 3) == 3) {
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) Q[a][b] = Q[a][b] + X[a][b];
+    }
+  }
+  const double f = 0.125 * coef;
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b <= a; b++) {
+      const zd v = scale(f, Q[a][b] - conj(Q[b][a]));
+      if (a == b) {
+        F[a * kCloverSites] = v.i;
+      } else {
+        F[(3 + 2 * (a + b - 1)) * kCloverSites] = v.r;
+        F[(4 + 2 * (a + b - 1)) * kCloverSites] = v.i;
+      }
     }
 }
 
@@ -398,9 +424,12 @@ __global__ void __launch_bounds__(128) k_field_strength(const void *u0, const vo
 __host__ __device__ constexpr int tri(int i, int j) { return i * (i + 1) / 2 + j; }
 __device__ inline zd hel(const zd (&M)[21], int i, int j) { return i >= j ? M[tri(i, j)] : conj(M[tri(j, i)]); }
 
-__device__ inline zd fplane(const double *F, long n, long j, int k, int a, int b) {
-  const double *p = F + (size_t)k * 18 * n;
-  return mk(p[(2 * (3 * a + b)) * n + j], p[(2 * (3 * a + b) + 1) * n + j]);
+// entry (a, b) of plane k of the field strength from the lane's LDS column
+__device__ inline zd fplane(const double *F, int k, int a, int b) {
+  const double *p = F + k * kPlaneReals * kCloverSites;
+  if (a == b) return mk(0.0, p[a * kCloverSites]);
+  const double re = p[(3 + 2 * (a + b - 1)) * kCloverSites], im = p[(4 + 2 * (a + b - 1)) * kCloverSites];
+  return a > b ? mk(re, im) : mk(-re, im);
 }
 
 // chiral block b of the clover term in Chroma's packing
@@ -408,13 +437,13 @@ __device__ inline zd fplane(const double *F, long n, long j, int k, int a, int b
 // with s = +1 (b = 0) or -1 (b = 1), G = i (F01 - s F23), H = (i F12 - F02) - s (i F03 + F13)
 //   A_b = [[diag_mass + G, H^+], [H, diag_mass - G]]
 // (F already carries the plane's clover coefficient)
-__device__ inline void clover_block(const double *F, long n, long j, int blk, double dm, zd (&A)[21]) {
+__device__ inline void clover_block(const double *F, int blk, double dm, zd (&A)[21]) {
   const double s = blk == 0 ? 1.0 : -1.0;
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
     for (int b = 0; b <= a; b++) {
-      const zd d = fplane(F, n, j, 0, a, b) - scale(s, fplane(F, n, j, 5, a, b));
+      const zd d = fplane(F, 0, a, b) - scale(s, fplane(F, 5, a, b));
       const zd g = mk(-d.i, d.r);
       A[tri(a, b)] = a == b ? mk(dm + g.r, 0.0) : g;
       A[tri(a + 3, b + 3)] = a == b ? mk(dm - g.r, 0.0) : scale(-1.0, g);
@@ -423,9 +452,9 @@ __device__ inline void clover_block(const double *F, long n, long j, int blk, do
   for (int a = 0; a < 3; a++)
 #pragma unroll
     for (int b = 0; b < 3; b++) {
-      const zd f2 = fplane(F, n, j, 2, a, b), f3 = fplane(F, n, j, 3, a, b);
-      const zd em = mk(-f2.i, f2.r) + fplane(F, n, j, 4, a, b);
-      const zd bm = mk(-f3.i, f3.r) - fplane(F, n, j, 1, a, b);
+      const zd f2 = fplane(F, 2, a, b), f3 = fplane(F, 3, a, b);
+      const zd em = mk(-f2.i, f2.r) + fplane(F, 4, a, b);
+      const zd bm = mk(-f3.i, f3.r) - fplane(F, 1, a, b);
       A[tri(a + 3, b)] = bm - scale(s, em);
     }
 }
@@ -489,19 +518,17 @@ __device__ inline void square_shift(zd (&A)[21], double shift) {
   for (int k = 0; k < 21; k++) A[k] = S[k];
 }
 
+constexpr bool clover_full(int what) { return what == 2 || what == 3 || what == 4; }
+
 // what: 0 A, 1 A^-1, 5 eps (A^2 + mu^2 - eps^2)^-1 (packed Hermitian, 36
 // reals per block); 2 (A + i mu g5)^-1 = (A^2 + mu^2)^-1 (A - i mu g5),
 // 3 (A^2 + mu^2 - eps^2)^-1 (A - i mu g5), 4 the same with + i mu g5 (full
-// complex blocks, 72 reals per block); results as FP64 into R[e * n + j]
-template <int WHAT>
-__global__ void __launch_bounds__(64) k_clover_block(const double *F, long n, double dm, double mu, double eps,
-                                                     double *R) {
-  const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int blk = blockIdx.y;
-  if (j >= n) return;
+// complex blocks, 72 reals per block); o(e, value) takes the reals of block blk
+template <int WHAT, typename Out>
+__device__ inline void clover_result(const double *F, int blk, double dm, double mu, double eps, Out o) {
   zd A[21];
-  clover_block(F, n, j, blk, dm, A);
-  if constexpr (WHAT == 0 || WHAT == 1 || WHAT == 5) {
+  clover_block(F, blk, dm, A);
+  if constexpr (!clover_full(WHAT)) {
     if constexpr (WHAT == 1) hpd_inverse(A);
     if constexpr (WHAT == 5) {
       square_shift(A, mu * mu - eps * eps);
@@ -509,25 +536,23 @@ __global__ void __launch_bounds__(64) k_clover_block(const double *F, long n, do
 #pragma unroll
       for (int k = 0; k < 21; k++) A[k] = scale(eps, A[k]);
     }
-    double *o = R + (size_t)36 * blk * n;
 #pragma unroll
-    for (int i = 0; i < 6; i++) o[i * n + j] = A[tri(i, i)].r;
+    for (int i = 0; i < 6; i++) o(i, A[tri(i, i)].r);
 #pragma unroll
     for (int i = 1; i < 6; i++)
 #pragma unroll
       for (int k = 0; k < i; k++) {
         const int e = i * (i - 1) / 2 + k;
-        o[(6 + 2 * e) * n + j] = A[tri(i, k)].r;
-        o[(6 + 2 * e + 1) * n + j] = A[tri(i, k)].i;
+        o(6 + 2 * e, A[tri(i, k)].r);
+        o(6 + 2 * e + 1, A[tri(i, k)].i);
       }
   } else {
     square_shift(A, WHAT == 2 ? mu * mu : mu * mu - eps * eps);
     hpd_inverse(A);  // A now holds N = (A^2 + shift)^-1
     zd B[21];
-    clover_block(F, n, j, blk, dm, B);  // the block again, for the factor on the right
+    clover_block(F, blk, dm, B);  // the block again, for the factor on the right
     const double g5 = blk == 0 ? 1.0 : -1.0;
     const double tw = (WHAT == 4 ? 1.0 : -1.0) * g5 * mu;
-    double *o = R + (size_t)72 * blk * n;
 #pragma unroll
     for (int i = 0; i < 6; i++)
 #pragma unroll
@@ -537,36 +562,74 @@ __global__ void __launch_bounds__(64) k_clover_block(const double *F, long n, do
         for (int q = 0; q < 6; q++) t = t + hel(A, i, q) * hel(B, q, k);
         const zd nik = hel(A, i, k);
         t = t + mk(-tw * nik.i, tw * nik.r);
-        o[(12 * i + 2 * k) * n + j] = t.r;
-        o[(12 * i + 2 * k + 1) * n + j] = t.i;
+        o(12 * i + 2 * k, t.r);
+        o(12 * i + 2 * k + 1, t.i);
       }
   }
 }
 
-// FP64 site values R[e * n + j] -> field of precision PO (sites s0 + j), one
-// word at a time (as store_all, including the FP16 per-site scale)
-template <int PO, int N>
-__global__ void k_clover_store(const double *R, long n, long s0, size_t vs, void *out) {
-  const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  typedef typename PT<PO>::calc T;
-  constexpr int pw = PT<PO>::per_word, nw = N / pw;
-  T inv = 1;
-  if constexpr (PT<PO>::scaled) {
-    float m = 0.f;
-    for (int e = 0; e < N; e++) m = fmaxf(m, fabsf((float)R[(size_t)e * n + j]));
-    inv = m > 0.f ? 1.0f / m : 0.f;
-    float *sc = reinterpret_cast<float *>(reinterpret_cast<char *>(out) + (size_t)nw * vs * 16);
-    sc[s0 + j] = m;
-  }
-  for (int w = 0; w < nw; w++) {
-    T v[pw];
-#pragma unroll
-    for (int k = 0; k < pw; k++) {
-      v[k] = (T)R[(size_t)(w * pw + k) * n + j];
-      if constexpr (PT<PO>::scaled) v[k] *= inv;
+// coef of plane 01 02 03 12 13 23: the planes with t take the temporal one
+template <int P, bool C12, int WHAT>
+__global__ void __launch_bounds__(2 * kCloverSites, 2) k_clover(const void *u0, const void *u1, size_t vs, Lat l, int cb,
+                                                             double cr, double ct, double dm, double mu, double eps,
+                                                             void *out) {
+  typedef typename PT<P>::calc T;
+  constexpr int N = clover_full(WHAT) ? kFullCloverReals : kCloverReals;  // reals per site
+  constexpr int pw = PT<P>::per_word, nw = N / pw;
+  // the half precisions scale a site's values by the largest of both blocks
+  // and pack eight to a word, so their blocks meet in LDS before the store
+  constexpr int kFBytes = 6 * kPlaneReals * kCloverSites * 8;
+  constexpr int kVBytes = PT<P>::scaled ? N * kCloverSites * 4 : 0;
+  __shared__ double lds[(kFBytes > kVBytes ? kFBytes : kVBytes) / 8];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const long s = (long)xcd_block() * kCloverSites + lane;
+  const bool live = s < l.vh;
+  double *F = lds + lane;
+  if (live) {
+    CloverSite x;
+    unsigned r = (unsigned)s;
+    const unsigned xh = r % (unsigned)l.nxh;
+    r /= (unsigned)l.nxh;
+    x.c1 = (int)(r % (unsigned)l.L[1]);
+    r /= (unsigned)l.L[1];
+    x.c2 = (int)(r % (unsigned)l.L[2]);
+    x.c3 = (int)(r / (unsigned)l.L[2]);
+    x.c0 = 2 * (int)xh + ((x.c1 + x.c2 + x.c3 + cb) & 1);
+#pragma nounroll
+    for (int k = 3 * wave; k < 3 * wave + 3; k++) {
+      const int pm = k < 3 ? 0 : k < 5 ? 1 : 2, pn = k < 3 ? k + 1 : k < 5 ? k - 1 : 3;
+      field_strength<P, C12>(u0, u1, vs, l, x, pm, pn, pn == 3 ? ct : cr, F + k * kPlaneReals * kCloverSites);
     }
-    Word<PO>::template store<false>(out, widx(s0 + j, w, nw), v);
+  }
+  __syncthreads();
+  if constexpr (!PT<P>::scaled) {
+    if (!live) return;
+    T v[N / 2];
+    clover_result<WHAT>(F, wave, dm, mu, eps, [&](int e, double x) { v[e] = (T)x; });
+#pragma unroll
+    for (int w = 0; w < nw / 2; w++) Word<P>::template store<false>(out, widx(s, wave * (nw / 2) + w, nw), v + w * pw);
+  } else {
+    float v[N / 2];
+    if (live) clover_result<WHAT>(F, wave, dm, mu, eps, [&](int e, double x) { v[e] = (float)x; });
+    __syncthreads();  // F is done with
+    float *V = reinterpret_cast<float *>(lds) + lane;
+    if (live) {
+#pragma unroll
+      for (int e = 0; e < N / 2; e++) V[(wave * (N / 2) + e) * kCloverSites] = v[e];
+    }
+    __syncthreads();
+    if (!live) return;
+    float m = 0.f;
+    for (int e = 0; e < N; e++) m = fmaxf(m, fabsf(V[e * kCloverSites]));
+    const float inv = m > 0.f ? 1.0f / m : 0.f;
+    if (wave == 0) reinterpret_cast<float *>(reinterpret_cast<char *>(out) + (size_t)nw * vs * 16)[s] = m;
+    for (int w = wave; w < nw; w += 2) {
+      float t[pw];
+#pragma unroll
+      for (int k = 0; k < pw; k++) t[k] = V[(w * pw + k) * kCloverSites] * inv;
+      Word<P>::template store<false>(out, widx(s, w, nw), t);
+    }
   }
 }
 
@@ -709,115 +772,22 @@ hipError_t fld_convert_clover(const GeomDesc &go, void *out, const GeomDesc &gi,
   return hipSuccess;
 }
 
-template <int P, bool C12, int MU, int NU>
-static void launch_fs(const GeomDesc &g, const Lat &l, const void *u0, const void *u1, int cb, long s0, long n,
-                      double coef, double *F, hipStream_t st) {
-  k_field_strength<P, C12, MU, NU><<<grid_for(n, 128), 128, 0, st>>>(u0, u1, g.vs, l, cb, s0, n, coef, F);
-}
-
-// all launches of one clover build, chunk by chunk, into the FP64 scratch
-// F (108 doubles per chunk site) and R (up to 144); stream-ordered, no
-// synchronisation
-template <int P, bool C12>
-static hipError_t clover_build_chunks(const GeomDesc &g, const void *u0, const void *u1, double cr, double ct,
-                                      double dm, int cb, int what, double mu, double eps, void *out, double *F,
-                                      double *R, long chunk, hipStream_t st) {
-  Lat l = make_lat(g);
-  const bool full = what == 2 || what == 3 || what == 4;
-  for (long s0 = 0; s0 < g.vh; s0 += chunk) {
-    const long n = (g.vh - s0) < chunk ? (g.vh - s0) : chunk;
-    // planes 01 02 03 12 13 23; the planes with t take the temporal coefficient
-    launch_fs<P, C12, 0, 1>(g, l, u0, u1, cb, s0, n, cr, F + 0 * 18 * n, st);
-    launch_fs<P, C12, 0, 2>(g, l, u0, u1, cb, s0, n, cr, F + 1 * 18 * n, st);
-    launch_fs<P, C12, 0, 3>(g, l, u0, u1, cb, s0, n, ct, F + 2 * 18 * n, st);
-    launch_fs<P, C12, 1, 2>(g, l, u0, u1, cb, s0, n, cr, F + 3 * 18 * n, st);
-    launch_fs<P, C12, 1, 3>(g, l, u0, u1, cb, s0, n, ct, F + 4 * 18 * n, st);
-    launch_fs<P, C12, 2, 3>(g, l, u0, u1, cb, s0, n, ct, F + 5 * 18 * n, st);
-    const dim3 gb((unsigned)((n + 63) / 64), 2);
-    switch (what) {
-      case 0: k_clover_block<0><<<gb, 64, 0, st>>>(F, n, dm, mu, eps, R); break;
-      case 1: k_clover_block<1><<<gb, 64, 0, st>>>(F, n, dm, mu, eps, R); break;
-      case 2: k_clover_block<2><<<gb, 64, 0, st>>>(F, n, dm, mu, eps, R); break;
-      case 3: k_clover_block<3><<<gb, 64, 0, st>>>(F, n, dm, mu, eps, R); break;
-      case 4: k_clover_block<4><<<gb, 64, 0, st>>>(F, n, dm, mu, eps, R); break;
-      default: k_clover_block<5><<<gb, 64, 0, st>>>(F, n, dm, mu, eps, R); break;
-    }
-    // output in the same precision as the gauge field
-    if (full)
-      k_clover_store<P, kFullCloverReals><<<grid_for(n), 256, 0, st>>>(R, n, s0, g.vs, out);
-    else
-      k_clover_store<P, kCloverReals><<<grid_for(n), 256, 0, st>>>(R, n, s0, g.vs, out);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
 template <int P, bool C12>
 static hipError_t clover_build_po(const GeomDesc &g, const void *u0, const void *u1, double cr, double ct, double dm,
                                   int cb, int what, double mu, double eps, void *out, hipStream_t st) {
-  // chunks of at most 2^20 sites bound the FP64 scratch (field strength 108,
-  // result up to 144 doubles per site) to about 2 GiB
-  const long chunk = g.vh < (1l << 20) ? g.vh : (1l << 20);
-  double *F = nullptr, *R = nullptr;
-  hipError_t e = hipMalloc(&F, sizeof(double) * 108 * (size_t)chunk);
-  if (e == hipSuccess) e = hipMalloc(&R, sizeof(double) * kFullCloverReals * (size_t)chunk);
-  if (e == hipSuccess) e = clover_build_chunks<P, C12>(g, u0, u1, cr, ct, dm, cb, what, mu, eps, out, F, R, chunk, st);
-  // the scratch is freed only after the stream has drained
-  const hipError_t es = hipStreamSynchronize(st);
-  if (F) (void)hipFree(F);
-  if (R) (void)hipFree(R);
-  return e != hipSuccess ? e : es;
-}
-// ---------------------------------------------------------------------------
-// allocation-free clover build
-//
-// `scratch` holds the FP64 field strength (108 doubles per site) and the
-// assembled blocks (up to 144 doubles per site) of kNoAllocSites sites; a
-// build of any lattice walks it in chunks of that many sites. Each device
-// holds its own copy of the array at its own address, looked up once per
-// device by fld_noalloc_init; host code passes only that address to kernels.
-// Every scratch entry a kernel reads is written earlier in the same call, so
-// nothing is cleared. Calls that overlap on one device share the array and race.
-// ---------------------------------------------------------------------------
-static __device__ __align__(256) double scratch[kNoAllocSites * (108 + kFullCloverReals)];
-static double *g_scratch_dev[kNoAllocMaxDevices] = {};
-
-hipError_t fld_noalloc_init(int device) {
-  if (device < 0 || device >= kNoAllocMaxDevices) return hipErrorInvalidDevice;
-  if (g_scratch_dev[device]) return hipSuccess;
-  double *p = nullptr;
-  const hipError_t e = hipGetSymbolAddress((void **)&p, HIP_SYMBOL(scratch));
-  if (e != hipSuccess) return e;
-  g_scratch_dev[device] = p;
-  return hipSuccess;
-}
-
-template <int P, bool C12>
-static hipError_t clover_build_noalloc_po(const GeomDesc &g, const void *u0, const void *u1, double cr, double ct,
-                                          double dm, int cb, int what, double mu, double eps, void *out,
-                                          double *scr, hipStream_t st) {
-  return clover_build_chunks<P, C12>(g, u0, u1, cr, ct, dm, cb, what, mu, eps, out, scr,
-                                     scr + 108 * kNoAllocSites, kNoAllocSites, st);
-}
-hipError_t fld_clover_build_noalloc(const GeomDesc &g, const void *u0, const void *u1, double cr, double ct,
-                                    double dm, int cb, int what, double mu, double eps, void *out, int device,
-                                    hipStream_t st) {
-  if (device < 0 || device >= kNoAllocMaxDevices || !g_scratch_dev[device]) return hipErrorNotInitialized;
-  double *scr = g_scratch_dev[device];
-  if (g.c12) {
-    PREC_SWITCH(g.prec, return (clover_build_noalloc_po<PP, true>(g, u0, u1, cr, ct, dm, cb, what, mu, eps, out,
-                                                                   scr, st)));
-  } else {
-    switch (g.prec) {
-      case P64: return clover_build_noalloc_po<P64, false>(g, u0, u1, cr, ct, dm, cb, what, mu, eps, out, scr, st);
-      case P32: return clover_build_noalloc_po<P32, false>(g, u0, u1, cr, ct, dm, cb, what, mu, eps, out, scr, st);
-      default: return hipErrorInvalidValue;
-    }
+  const Lat l = make_lat(g);
+  const dim3 grid = grid_for(g.vh, kCloverSites);
+  switch (what) {
+#define CK(W) \
+  case W: k_clover<P, C12, W><<<grid, 2 * kCloverSites, 0, st>>>(u0, u1, g.vs, l, cb, cr, ct, dm, mu, eps, out); break;
+    CK(0) CK(1) CK(2) CK(3) CK(4) CK(5)
+#undef CK
+    default: return hipErrorInvalidValue;
   }
-  return hipSuccess;
+  return hipGetLastError();
 }
 
+// one launch, stream-ordered: no scratch, allocation or synchronisation
 hipError_t fld_clover_build(const GeomDesc &g, const void *u0, const void *u1, double cr, double ct, double dm,
                             int cb, int what, double mu, double eps, void *out, hipStream_t st) {
   if (g.c12) {
