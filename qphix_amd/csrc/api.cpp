@@ -815,6 +815,7 @@ static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, 
         if (bz <= g.L[2] && g.L[2] % bz == 0 && g.L[3] % sl == 0 && g.L[3] / sl >= 2)
           cand.push_back({blk, bz, sl, 0, 1, 1});
   }
+  if (kind != KD_DIR) cand.push_back({256, -1, 1, 0, 1, 1});  // the eight terms over wavefronts
   DevBuf scratch;
   if (hipMalloc(&scratch.p, spinor_bytes(g)) != hipSuccess) {
     (void)hipGetLastError();
@@ -891,6 +892,7 @@ static void tune_rhs_tile(const GeomDesc &g, int kind, int isign, const HopArgs 
   // first the tiling under the single-RHS traversal; the matrix-core form
   // (reg 8) is not a candidate: it runs slower per source than the register
   // tiles (qphix_tune_rhs(8, n) still forces it)
+  if (cfg.bz < 0) cfg.bz = 0;  // a register tile has no split form
   a.bz = cfg.bz;
   a.slabs = cfg.slabs;
   std::vector<HopCfg> tiles;

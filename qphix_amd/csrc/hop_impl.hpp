@@ -39,7 +39,8 @@ struct HopArgs {
   double tbc_r[4], tbc_i[4];
   int tbc_mask;
   double alpha, mu, muinv, rho;
-  // traversal: bz = 0 is the natural site order; otherwise the (y, z) cross
+  // traversal: bz = 0 is the natural site order, bz < 0 too, with the eight
+  // terms of a site split over wavefronts (hop_split.hpp); otherwise the (y, z) cross
   // section is cut into tiles of by rows (by = 0: all of y) by bz planes and
   // each of `slabs` t-slabs is walked tile by tile, t innermost, so consecutive
   // work-groups of one XCD reuse the source spinor slices they share
@@ -130,10 +131,10 @@ template <int P, bool C12> struct GaugeLayout {
 // blocks and stop the scheduler from issuing the next hop's loads early.
 // apply_hop_h takes the projected half spinor h = (1 -/+ isign g_mu) psi.
 // FMA: the link products as FMA chains (cmul_f / cfma; FP16 storage)
-template <int MU, int S, bool FWD, bool C12, bool FMA = false, typename T>
-__device__ inline void apply_hop_h(const cx<T> (&U)[3][3], const cx<T> (&h)[2][3], T coef, T tr, T ti,
-                                   cx<T> (&acc)[4][3]) {
-  cx<T> uh[2][3];
+// uh = phase U h (or U^+ h)
+template <bool FWD, bool FMA, typename T>
+__device__ inline void link_times_half(const cx<T> (&U)[3][3], const cx<T> (&h)[2][3], T tr, T ti,
+                                       cx<T> (&uh)[2][3]) {
 #pragma unroll
   for (int r = 0; r < 2; r++)
 #pragma unroll
@@ -163,6 +164,12 @@ __device__ inline void apply_hop_h(const cx<T> (&U)[3][3], const cx<T> (&h)[2][3
   for (int r = 0; r < 2; r++)
 #pragma unroll
     for (int i = 0; i < 3; i++) uh[r][i] = ph * uh[r][i];
+}
+template <int MU, int S, bool FWD, bool C12, bool FMA = false, typename T>
+__device__ inline void apply_hop_h(const cx<T> (&U)[3][3], const cx<T> (&h)[2][3], T coef, T tr, T ti,
+                                   cx<T> (&acc)[4][3]) {
+  cx<T> uh[2][3];
+  link_times_half<FWD, FMA>(U, h, tr, ti, uh);
   recon_acc<MU, S>(acc, uh, coef);
 }
 
@@ -329,10 +336,11 @@ __device__ inline void herm6(const T *m, const cx<T> (&in)[6], cx<T> (&out)[6]) 
   }
 }
 
-template <bool FMA = false, typename T>
-__device__ inline void full6(const T *m, const cx<T> (&in)[6], cx<T> (&out)[6]) {
+// rows of out = M in for a full complex block m (NR of its six rows)
+template <bool FMA = false, int NR, typename T>
+__device__ inline void full6_rows(const T *m, const cx<T> (&in)[6], cx<T> (&out)[NR]) {
 #pragma unroll
-  for (int i = 0; i < 6; i++) {
+  for (int i = 0; i < NR; i++) {
     cx<T> s;
     if constexpr (FMA) s = cmul_f(mk(m[12 * i], m[12 * i + 1]), in[0]);
     else s = mk(m[12 * i], m[12 * i + 1]) * in[0];
@@ -343,6 +351,10 @@ __device__ inline void full6(const T *m, const cx<T> (&in)[6], cx<T> (&out)[6]) 
     }
     out[i] = s;
   }
+}
+template <bool FMA = false, typename T>
+__device__ inline void full6(const T *m, const cx<T> (&in)[6], cx<T> (&out)[6]) {
+  full6_rows<FMA>(m, in, out);
 }
 
 template <int P, int B, typename T>

@@ -2,12 +2,24 @@
 #pragma once
 
 #include "hop_impl.hpp"
+#include "hop_split.hpp"
 
 namespace qphix_amd {
 
 template <int P, bool C12, int ISIGN>
 static hipError_t launch_hop3(int kind, const HopArgs &a, int block, hipStream_t st) {
   const int nr = a.nrhs > 1 ? a.nrhs : 1;
+  if (use_split(P, kind, a, nr)) {
+    const dim3 grid((unsigned)(((a.vh + kSplitSites - 1) / kSplitSites) * nr));
+    switch (kind) {
+#define SK(K) \
+  case K: hop_split_kernel<P, C12, ISIGN, K><<<grid, split_threads(P, K), 0, st>>>(a); break;
+      SK(KD_WILSON) SK(KA_WILSON) SK(KD_CLOVER) SK(KA_CLOVER) SK(KD_TM) SK(KA_TM) SK(KD_FULL)
+#undef SK
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   const dim3 grid((unsigned)(((a.vh + block - 1) / block) * nr));
   switch (kind) {
     case KD_WILSON: hop_kernel<P, C12, ISIGN, KD_WILSON><<<grid, block, a.lds_cap, st>>>(a); break;
