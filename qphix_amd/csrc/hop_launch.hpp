@@ -13,7 +13,7 @@ static hipError_t launch_hop3(int kind, const HopArgs &a, int block, hipStream_t
     const dim3 grid((unsigned)(((a.vh + kSplitSites - 1) / kSplitSites) * nr));
     switch (kind) {
 #define SK(K) \
-  case K: hop_split_kernel<P, C12, ISIGN, K><<<grid, split_threads(P, K), 0, st>>>(a); break;
+  case K: hop_split_kernel<P, C12, ISIGN, K><<<grid, split_threads(K), 0, st>>>(a); break;
       SK(KD_WILSON) SK(KA_WILSON) SK(KD_CLOVER) SK(KA_CLOVER) SK(KD_TM) SK(KA_TM) SK(KD_FULL)
 #undef SK
       default: return hipErrorInvalidValue;

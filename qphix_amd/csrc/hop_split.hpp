@@ -16,10 +16,14 @@
 namespace qphix_amd {
 
 constexpr int kSplitSites = 64;
-// wavefronts of the epilogue: one per chiral block; one per spin where a full
-// FP64 block (144 registers) would not fit beside the sums
-constexpr int split_epi(int p, int kind) { return p == P64 && kind == KD_FULL ? 4 : 2; }
-constexpr int split_threads(int p, int kind) { return 64 * (8 + split_epi(p, kind)); }
+// wavefronts of the epilogue: one per chiral block, or one per spin for the
+// full blocks, whose registers (72 or 144) would cost half the work-groups
+constexpr int split_epi(int kind) { return kind == KD_FULL ? 4 : 2; }
+constexpr int split_threads(int kind) { return 64 * (8 + split_epi(kind)); }
+// the results meet in LDS before the store: the half precisions scale a site's
+// values by the largest of them, and a spin of FP32 is a word and a half
+constexpr bool split_gather(int p, int kind) { return p == P16 || p == PB16 || (p == P32 && kind == KD_FULL); }
+
 
 // Largest number of sites (times right-hand sides) that take this form by
 // rule; from 2^17 sites on, where the hops are tuned, it is a candidate of the
@@ -29,7 +33,8 @@ constexpr int split_threads(int p, int kind) { return 64 * (8 + split_epi(p, kin
 // 49152 20.6 / 19.6, 65536 23.8 / 24.8; FP32 2048 7.5 / 4.2, 32768 12.4 / 5.3,
 // 96000 18.9 / 15.6, 331776 51.8 / 48.5; FP16 2048 7.1 / 4.7, 32768 8.4 / 5.8,
 // 49152 9.3 / 8.0, 65536 9.7 / 11.3 (Wilson 7.45 / 7.62 at 49152). Full
-// blocks in FP32: 49152 14.2 / 12.5, 65536 15.6 / 15.7.
+// blocks in FP32: 32768 13.4 / 7.3, 49152 14.2 / 12.2, 65536 15.6 / 15.5; in
+// FP16: 32768 9.8 / 5.6.
 constexpr long split_sites(int p, int kind) {
   return p == P64 ? 49152 : p == P32 ? (kind == KD_FULL ? 49152 : (1l << 17) - 1) : 45056;
 }
@@ -235,9 +240,9 @@ __device__ inline void split_epilogue(const HopArgs &a, const typename PT<P>::ca
         o[6 * q + 2 * c + 1] = x[q][c].i;
       }
   }
-  if constexpr (raw) {  // both blocks meet in LDS for the site's scale
+  if constexpr (split_gather(P, KIND)) {
 #pragma unroll
-    for (int k = 0; k < 12; k++) res[(12 * B + k) * kSplitSites] = o[k];
+    for (int k = 0; k < 2 * rows; k++) res[(12 * B + 2 * row0 + k) * kSplitSites] = o[k];
   } else {
     constexpr int pw = PT<P>::per_word, w0 = (12 * B + 2 * row0) / pw;
 #pragma unroll
@@ -245,12 +250,18 @@ __device__ inline void split_epilogue(const HopArgs &a, const typename PT<P>::ca
   }
 }
 
+// three work-groups of ten wavefronts to a CU (64 registers) where a spill-free
+// allocation gives them
+constexpr int split_min_waves(int p, int kind) {
+  return (p == P16 || p == PB16) && kind != KD_FULL && kind != KD_CLOVER ? 8 : 1;
+}
+
 template <int P, bool C12, int ISIGN, int KIND>
-__global__ void __launch_bounds__(split_threads(P, KIND)) hop_split_kernel(const HopArgs a) {
+__global__ void __launch_bounds__(split_threads(KIND), split_min_waves(P, KIND)) hop_split_kernel(const HopArgs a) {
   if (a.skip && *a.skip) return;
   typedef typename PT<P>::calc T;
   __shared__ T terms[8 * 12 * kSplitSites];
-  __shared__ T result[PT<P>::scaled ? 24 * kSplitSites : 1];
+  __shared__ T result[split_gather(P, KIND) ? 24 * kSplitSites : 1];
   int lb = xcd_block();
   const void *psi_p = a.psi, *chi_p = a.chi;
   void *out_p = a.out;
@@ -266,7 +277,7 @@ __global__ void __launch_bounds__(split_threads(P, KIND)) hop_split_kernel(const
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const unsigned s = (unsigned)lb * kSplitSites + lane;
   const bool live = s < (unsigned)a.vh;
-  T *res = result + (PT<P>::scaled ? lane : 0);
+  T *res = result + (split_gather(P, KIND) ? lane : 0);
   if (wave < 8) {
     if (live) {
       T *lds = terms + wave * 12 * kSplitSites + lane;
@@ -284,7 +295,7 @@ __global__ void __launch_bounds__(split_threads(P, KIND)) hop_split_kernel(const
       }
     }
     __syncthreads();
-  } else if constexpr (split_epi(P, KIND) == 2) {
+  } else if constexpr (split_epi(KIND) == 2) {
     if (wave == 8) split_epilogue<P, ISIGN, KIND, 0, -1>(a, terms + lane, res, chi_p, out_p, s, live);
     else split_epilogue<P, ISIGN, KIND, 1, -1>(a, terms + lane, res, chi_p, out_p, s, live);
   } else {
@@ -293,19 +304,24 @@ __global__ void __launch_bounds__(split_threads(P, KIND)) hop_split_kernel(const
     else if (wave == 10) split_epilogue<P, ISIGN, KIND, 1, 0>(a, terms + lane, res, chi_p, out_p, s, live);
     else split_epilogue<P, ISIGN, KIND, 1, 1>(a, terms + lane, res, chi_p, out_p, s, live);
   }
-  if constexpr (PT<P>::scaled) {
+  if constexpr (split_gather(P, KIND)) {
     __syncthreads();
     if (wave < words_of<P>(kSpinorReals) && live) {  // a word per wavefront, as store_all
       constexpr int pw = PT<P>::per_word, nws = words_of<P>(kSpinorReals);
-      float m = 0.f;
+      T t[pw];
+      if constexpr (PT<P>::scaled) {
+        float m = 0.f;
 #pragma unroll
-      for (int k = 0; k < kSpinorReals; k++) m = fmaxf(m, fabsf(res[k * kSplitSites]));
-      const float inv = m > 0.f ? 1.0f / m : 0.f;
-      float t[pw];
+        for (int k = 0; k < kSpinorReals; k++) m = fmaxf(m, fabsf(res[k * kSplitSites]));
+        const float inv = m > 0.f ? 1.0f / m : 0.f;
 #pragma unroll
-      for (int k = 0; k < pw; k++) t[k] = res[(wave * pw + k) * kSplitSites] * inv;
+        for (int k = 0; k < pw; k++) t[k] = res[(wave * pw + k) * kSplitSites] * inv;
+        if (wave == 0) reinterpret_cast<float *>(reinterpret_cast<char *>(out_p) + (size_t)nws * a.vs * 16)[s] = m;
+      } else {
+#pragma unroll
+        for (int k = 0; k < pw; k++) t[k] = res[(wave * pw + k) * kSplitSites];
+      }
       Word<P>::template store<true>(out_p, widx(s, wave, nws), t);
-      if (wave == 0) reinterpret_cast<float *>(reinterpret_cast<char *>(out_p) + (size_t)nws * a.vs * 16)[s] = m;
     }
   }
 }
