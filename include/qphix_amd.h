@@ -357,9 +357,9 @@ int qphix_minvcg_set_mode(qphix_solver *s, int mode);
 /* The same control for CG and BiCGStab solvers (no reference counterpart;
  * the reference keeps their scalars on the host, invcg.h:293-343,
  * invbicgstab.h:150-256) and for multishift CG (as qphix_minvcg_set_mode). CG
- * and BiCGStab default to 0; modes 1 and 2 apply to single-flavour operators
- * and silent solves (the others run mode 0) and give bit-identical solutions,
- * counters and statuses. */
+ * and BiCGStab default to 1; modes 1 and 2 apply to single-flavour operators
+ * and silent solves (the others run mode 0); all three give bit-identical
+ * solutions, counters and statuses. */
 int qphix_solver_set_mode(qphix_solver *s, int mode);
 /* x[shift * nflav + f]; rsd_sq_final[n_shift] */
 int qphix_minvcg_solve(qphix_solver *s, void *const x[], const void *const rhs[],

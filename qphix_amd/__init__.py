@@ -426,7 +426,7 @@ class Solver:
 
     def set_mode(self, mode):
         """0 host scalars, 1 device scalars, 2 device scalars with the
-        iteration replayed from a HIP graph (BiCGStab and multishift CG)."""
+        iteration replayed from a HIP graph (CG, BiCGStab, multishift CG)."""
         call("qphix_solver_set_mode", self.h, mode)
         return self
 

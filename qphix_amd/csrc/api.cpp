@@ -88,9 +88,13 @@ struct qphix_solver {
   // FP64 scalars in device memory with eager launches, 2 the same with each
   // iteration replayed from a HIP graph
   int ms_mode = 2;
-  // BiCGStab control: 0 host scalars, 1 device scalars (eager launches), 2
-  // device scalars with the iteration replayed from a HIP graph
-  int dev_mode = 0;
+  // CG and BiCGStab control: 0 host scalars, 1 device scalars (eager
+  // launches), 2 device scalars with the iteration replayed from a HIP graph.
+  // 1 is the fastest at every size measured (8^4 FP64 CG to 1e-12: 2.37, 1.75
+  // and 1.94 ms; 24^3x48: 23.9, 23.3 and 23.6 ms): no wait per reduction, and
+  // no graph to build per solve
+  int dev_mode = 1;
+  void *dstate = nullptr;  // their device state, from the first solve on
 };
 
 // ---------------------------------------------------------------------------
@@ -102,6 +106,7 @@ static int g_device = 0;
 static hipStream_t g_own_stream = nullptr;
 static hipStream_t g_stream = nullptr;
 static double *g_partials = nullptr;  // device, kMaxBlasBlocks * 3
+static unsigned *g_tickets = nullptr;  // device, the reductions' work-group counters
 static double *g_dres = nullptr;      // device, kResults
 static double *g_hres = nullptr;      // pinned host, kResults
 static constexpr int kResults = 4 * kMaxRhs;
@@ -167,6 +172,8 @@ extern "C" int qphix_init(int device) {
   HIPCHK(hipStreamCreate(&g_own_stream));
   g_stream = g_own_stream;
   HIPCHK(hipMalloc(&g_partials, sizeof(double) * kMaxBlasBlocks * 3));
+  HIPCHK(hipMalloc(&g_tickets, sizeof(unsigned) * kTickets));
+  HIPCHK(hipMemset(g_tickets, 0, sizeof(unsigned) * kTickets));
   HIPCHK(hipMalloc(&g_dres, sizeof(double) * kResults));
   HIPCHK(hipHostMalloc(&g_hres, sizeof(double) * kResults, hipHostMallocDefault));
   HIPCHK(hipEventCreate(&g_ev0));
@@ -448,13 +455,14 @@ extern "C" int qphix_clover_build_noalloc(const qphix_geom *g, const void *u0, c
 // ---------------------------------------------------------------------------
 // BLAS plumbing
 // ---------------------------------------------------------------------------
+static BlasFin blas_fin(double *out, int tail = TAIL_NONE, void *state = nullptr) {
+  return BlasFin{g_partials, g_tickets, out, tail, state};
+}
+// the sums go straight to pinned host memory; the wait is for the kernel alone
 static int run_blas(const qphix_geom *g, int op, const BlasArgs &a, double *out) {
-  int nb = 0;
-  HIPCHK(blas_launch(g->d, op, a, g_partials, &nb, g_stream));
+  HIPCHK(blas_launch(g->d, op, a, blas_fin(g_hres), g_stream));
   const int nr = blas_nred(op);
   if (nr > 0) {
-    HIPCHK(blas_finalize(g_partials, nb, nr, g_dres, g_stream));
-    HIPCHK(hipMemcpyAsync(g_hres, g_dres, nr * sizeof(double), hipMemcpyDeviceToHost, g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
     if (out)
       for (int k = 0; k < nr; k++) out[k] = g_hres[k];
@@ -497,9 +505,7 @@ extern "C" int qphix_stream_calibrate(const qphix_geom *g, int words_in, int wor
 // the reduction left in device memory: kernels only (no copy, no memset, no
 // synchronisation), so the call can be captured in a HIP graph
 static int run_blas_dev(const qphix_geom *g, int op, const BlasArgs &a, double *d_out) {
-  int nb = 0;
-  HIPCHK(blas_launch(g->d, op, a, g_partials, &nb, g_stream));
-  HIPCHK(blas_finalize(g_partials, nb, blas_nred(op), d_out, g_stream));
+  HIPCHK(blas_launch(g->d, op, a, blas_fin(d_out), g_stream));
   return QPHIX_OK;
 }
 static BlasArgs bargs() {
@@ -1579,6 +1585,7 @@ extern "C" int qphix_solver_destroy(qphix_solver *s) {
   if (!s) return QPHIX_OK;
   for (void *p : s->work) qphix_free(p);
   for (void *p : s->mwork) qphix_free(p);
+  qphix_free(s->dstate);
   delete s;
   return QPHIX_OK;
 }
@@ -1589,7 +1596,8 @@ extern "C" int qphix_solver_destroy(qphix_solver *s) {
 // when x is exactly zero.  On convergence the reference leaves rsd_sq_final
 // unset; here it is the recursively updated |r|^2 (absolute), the quantity the
 // convergence test used.
-static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc, double *d_out);
+static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc, double *d_out = nullptr,
+                      int tail = TAIL_NONE, void *state = nullptr);
 static int cg_device_loop(qphix_solver *s, void *x, const SV &r, const SV &p, SV &mp, SV &mmp, int isign, int cb,
                           double cp, double rsd_sq, unsigned long sf, qphix_solve_stats *st);
 
@@ -1677,13 +1685,33 @@ static int solve_cg(qphix_solver *s, void *const *x, const void *const *rhs, dou
 }
 
 // a BLAS step whose scalars come from device memory (dsc; BlasArgs::dsc), its
-// reduction (if any) finalized into device memory: kernels only
-static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc, double *d_out) {
+// reduction (if any) ending in device memory with a solver's scalar step
+static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc, double *d_out, int tail,
+                      void *state) {
   a.dsc = dsc;
-  int nb = 0;
-  HIPCHK(blas_launch(g->d, op, a, g_partials, &nb, g_stream));
-  if (blas_nred(op) > 0) HIPCHK(blas_finalize(g_partials, nb, blas_nred(op), d_out, g_stream));
+  HIPCHK(blas_launch(g->d, op, a, blas_fin(d_out, tail, state), g_stream));
   return QPHIX_OK;
+}
+
+// the device state of a solver's device-resident loop (S: its type)
+template <typename S> static int solver_state(qphix_solver *s, S **st) {
+  if (!s->dstate) {
+    const size_t n = std::max(std::max(sizeof(BiState), sizeof(CgDState)), sizeof(MsState));
+    if (hipMalloc(&s->dstate, n) != hipSuccess) {
+      (void)hipGetLastError();
+      s->dstate = nullptr;
+      return fail(QPHIX_ENOMEM, "solver state allocation");
+    }
+  }
+  *st = (S *)s->dstate;
+  return QPHIX_OK;
+}
+// nothing published yet (no kernel of a loop is in flight)
+static void clear_view(SolverView *v) {
+  for (int k = 0; k < 2; k++) {
+    v[k].done = 0;
+    v[k].progress = 0;
+  }
 }
 
 struct GraphRun {
@@ -1745,8 +1773,8 @@ static int device_iterations(int mode, int max_steps, const std::function<int()>
 
 // The BiCGStab iteration (single flavour) with its scalars in device memory
 // (BiState): p-update, v = M p, <r0, v>, s-update, t = M r, <t, r> and |t|^2,
-// the x/r update with |r|^2 and <r0, r>, between them four single-thread
-// kernels with the host loop's scalar arithmetic; no host round trip
+// the x/r update with |r|^2 and <r0, r>; the scalar arithmetic of the host loop
+// is taken where each reduction ends (BlasTail), with no host round trip
 // (device_iterations runs it). Iterations after the end only read: the vector
 // updates and the hops skip themselves.
 static int bicgstab_device_loop(qphix_solver *s, void *x, const SV &r0, const SV &r, const SV &p, SV &v, SV &t,
@@ -1768,39 +1796,35 @@ static int bicgstab_device_loop(qphix_solver *s, void *x, const SV &r0, const SV
   h.max_iters = s->max_iters;
   h.progress = r_norm / rsd_sq;
   h.hview = g_bi_view;
-  DevBuf dbs;
-  if (hipMalloc(&dbs.p, sizeof(BiState)) != hipSuccess) return fail(QPHIX_ENOMEM, "BiCGStab state allocation");
-  BiState *bs = (BiState *)dbs.p;
-  HIPCHK(hipMemcpyAsync(bs, &h, sizeof(h), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
+  BiState *bs;
+  TRY(solver_state(s, &bs));
+  clear_view(g_bi_view);
+  HIPCHK(bi_set_launch(bs, h, g_stream));
   struct SkipScope {  // hop launches of this loop skip once the solve is done
     explicit SkipScope(const int *p) { g_hop_skip = p; }
     ~SkipScope() { g_hop_skip = nullptr; }
   } skip_scope(&bs->done);
   auto iteration = [&]() -> int {
-    HIPCHK(bi_pre_launch(bs, g_stream));
     BlasArgs a = bargs();
     a.x = r[0]; a.y = v[0]; a.o0 = p[0];
-    TRY(run_blas_q(g, B_PUPD, a, bs->pupd, nullptr));
+    TRY(run_blas_q(g, B_PUPD, a, bs->pupd));
     TRY(op_apply_v(M, v, cv(p), isign, cb));
     a = bargs();
     a.x = r0[0]; a.y = v[0];
-    TRY(run_blas_q(g, B_CDOT, a, nullptr, bs->r0v));
-    HIPCHK(bi_mid_launch(bs, g_stream));
+    TRY(run_blas_q(g, B_CDOT, a, nullptr, bs->r0v, TAIL_BI_MID, bs));
     a = bargs();
     a.x = v[0]; a.o0 = r[0];
-    TRY(run_blas_q(g, B_SUPD, a, bs->supd, nullptr));
+    TRY(run_blas_q(g, B_SUPD, a, bs->supd));
     TRY(op_apply_v(M, t, cv(r), isign, cb));
     a = bargs();
     a.x = t[0]; a.y = r[0];
-    TRY(run_blas_q(g, B_CDOTNORM, a, nullptr, bs->tr));
-    HIPCHK(bi_mid2_launch(bs, g_stream));
+    TRY(run_blas_q(g, B_CDOTNORM, a, nullptr, bs->tr, TAIL_BI_MID2, bs));
     a = bargs();
     a.x = t[0]; a.y = p[0]; a.z = r0[0]; a.o0 = x; a.o1 = r[0];
-    TRY(run_blas_q(g, B_RXUPD_CDOT, a, bs->rxupd, bs->ru));
-    HIPCHK(bi_post_launch(bs, g_stream));
+    TRY(run_blas_q(g, B_RXUPD_CDOT, a, bs->rxupd, bs->ru, TAIL_BI_POST, bs));
     return QPHIX_OK;
   };
+  HIPCHK(bi_pre_launch(bs, g_stream));
   TRY(device_iterations(s->dev_mode, s->max_iters + 1, iteration, g_bi_view));
   HIPCHK(hipMemcpyAsync(&h, bs, sizeof(h), hipMemcpyDeviceToHost, g_stream));
   HIPCHK(hipStreamSynchronize(g_stream));
@@ -1813,8 +1837,8 @@ static int bicgstab_device_loop(qphix_solver *s, void *x, const SV &r0, const SV
 }
 
 // The CG iteration on M^+M (single flavour) with its scalars in device memory
-// (CgDState): M^+M p, |M p|^2, a (k_cgd_mid), r -= a M^+M p and x += a p with
-// |r|^2, the convergence test and b (k_cgd_post), p = b p + r; no host round trip.
+// (CgDState): M^+M p, |M p|^2 and a, r -= a M^+M p and x += a p with |r|^2, the
+// convergence test and b, p = b p + r; no host round trip.
 static SolverView *g_cg_view = nullptr;  // pinned host, 2 entries
 static int cg_device_loop(qphix_solver *s, void *x, const SV &r, const SV &p, SV &mp, SV &mmp, int isign, int cb,
                           double cp, double rsd_sq, unsigned long sf, qphix_solve_stats *st) {
@@ -1832,11 +1856,10 @@ static int cg_device_loop(qphix_solver *s, void *x, const SV &r, const SV &p, SV
   h.max_iters = s->max_iters;
   h.progress = cp / rsd_sq;
   h.hview = g_cg_view;
-  DevBuf dcs;
-  if (hipMalloc(&dcs.p, sizeof(CgDState)) != hipSuccess) return fail(QPHIX_ENOMEM, "CG state allocation");
-  CgDState *cs = (CgDState *)dcs.p;
-  HIPCHK(hipMemcpyAsync(cs, &h, sizeof(h), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
+  CgDState *cs;
+  TRY(solver_state(s, &cs));
+  clear_view(g_cg_view);
+  HIPCHK(cgd_set_launch(cs, h, g_stream));
   struct SkipScope {  // hop launches of this loop skip once the solve is done
     explicit SkipScope(const int *q) { g_hop_skip = q; }
     ~SkipScope() { g_hop_skip = nullptr; }
@@ -1846,15 +1869,13 @@ static int cg_device_loop(qphix_solver *s, void *x, const SV &r, const SV &p, SV
     TRY(op_apply_v(M, mmp, cv(mp), -isign, cb));
     BlasArgs a = bargs();
     a.x = mp[0];
-    TRY(run_blas_q(g, B_NORM2, a, nullptr, &cs->d_raw));
-    HIPCHK(cgd_mid_launch(cs, g_stream));
+    TRY(run_blas_q(g, B_NORM2, a, nullptr, &cs->d_raw, TAIL_CG_MID, cs));
     a = bargs();
     a.x = mmp[0]; a.y = p[0]; a.o0 = r[0]; a.o1 = x;
-    TRY(run_blas_q(g, B_RMAMMP, a, cs->rmammp, &cs->r_raw));
-    HIPCHK(cgd_post_launch(cs, g_stream));
+    TRY(run_blas_q(g, B_RMAMMP, a, cs->rmammp, &cs->r_raw, TAIL_CG_POST, cs));
     a = bargs();
     a.x = r[0]; a.o0 = p[0];
-    TRY(run_blas_q(g, B_AYPX, a, cs->aypx, nullptr));
+    TRY(run_blas_q(g, B_AYPX, a, cs->aypx));
     return QPHIX_OK;
   };
   TRY(device_iterations(s->dev_mode, s->max_iters + 1, iteration, g_cg_view));
@@ -2716,13 +2737,12 @@ extern "C" int qphix_solve_multi(qphix_solver *s, void *const x[], const void *c
   return QPHIX_OK;
 }
 
-// The multishift iteration with its scalars in device memory (MsState): per
-// iteration the kernels a / as_s (k_ms_pre), the vector sweep, M^+M p0, |M p0|^2,
-// b (k_ms_mid), r += b M^+M p0 with |r|^2, then the zeta / beta recurrences and
-// the convergence test (k_ms_post); no host round trip (device_iterations runs
-// it, eagerly or replayed from a HIP graph). Once done the state is frozen; a
-// closing sweep applies the x_s updates left pending. Returns 0, -1 (not
-// converged) or a status.
+// The multishift iteration with its scalars in device memory (MsState): the
+// vector sweep, M^+M p0, |M p0|^2 and b, r += b M^+M p0 with |r|^2, the zeta /
+// beta recurrences, the convergence test and the next iteration's a, as_s
+// (BlasTail); no host round trip (device_iterations runs it, eagerly or replayed
+// from a HIP graph). Once done the state is frozen; a closing sweep applies
+// the x_s updates left pending. Returns 0, -1 (not converged) or a status.
 static SolverView *g_ms_view = nullptr;  // pinned host, 2 entries
 static int device_iterations(int mode, int max_steps, const std::function<int()> &iteration,
                              SolverView *view);
@@ -2757,11 +2777,10 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
     h.beta[q] = beta[q];
     h.rsd_sq[q] = rsd_sq[q];
   }
-  DevBuf dms;
-  if (hipMalloc(&dms.p, sizeof(MsState)) != hipSuccess) return fail(QPHIX_ENOMEM, "multishift state allocation");
-  MsState *ms = (MsState *)dms.p;
-  HIPCHK(hipMemcpyAsync(ms, &h, sizeof(h), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
+  MsState *ms;
+  TRY(solver_state(s, &ms));
+  clear_view(g_ms_view);
+  HIPCHK(ms_set_launch(ms, h, g_stream));
   auto sweep = [&]() -> int {
     for (int f = 0; f < nf; f++) {
       MShiftArgs m;
@@ -2788,18 +2807,16 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
     for (int f = 0; f < nf; f++) {
       BlasArgs a = bargs();
       a.x = mp[f];
-      TRY(run_blas_dev(g, B_NORM2, a, &ms->cf[f]));
+      TRY(run_blas_q(g, B_NORM2, a, nullptr, &ms->cf[f], f + 1 == nf ? TAIL_MS_MID : TAIL_NONE, ms));
     }
-    HIPCHK(ms_mid_launch(ms, g_stream));
     for (int f = 0; f < nf; f++)
-      HIPCHK(axpy_norm2_dev_launch(g->d, &ms->b, mmp[f], r[f], g_partials, &ms->cf[f], g_stream));
-    HIPCHK(ms_post_launch(ms, g_stream));
+      HIPCHK(axpy_norm2_dev_launch(g->d, &ms->b, mmp[f], r[f],
+                                   blas_fin(&ms->cf[f], f + 1 == nf ? TAIL_MS_POST : TAIL_NONE, ms), g_stream));
     return QPHIX_OK;
   };
   HIPCHK(ms_pre_launch(ms, g_stream));  // the first iteration's a, as_s
   TRY(device_iterations(s->ms_mode, s->max_iters, iteration, g_ms_view));
   TRY(sweep());  // the pending x_s updates (a no-op if the last iteration applied them)
-  HIPCHK(ms_post_launch(ms, g_stream));
   HIPCHK(hipMemcpyAsync(&h, ms, sizeof(h), hipMemcpyDeviceToHost, g_stream));
   HIPCHK(hipStreamSynchronize(g_stream));
   *n_iters = h.iters;

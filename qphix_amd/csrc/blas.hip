@@ -5,9 +5,11 @@
 // operands, updates them in the geometry's arithmetic type (float for F32 and
 // F16 storage, as ArithType<half> = float in the reference) and accumulates up
 // to three reductions in double. Reductions are combined by a wavefront
-// shuffle tree, then across the waves of the block through LDS, and the
-// per-block partials are summed in a fixed order by a one-block finalize
-// kernel, so results are bitwise reproducible for a given lattice.
+// shuffle tree, then across the waves of the block through LDS, and the last
+// block to finish sums the per-block partials in a fixed order, so results are
+// bitwise reproducible for a given lattice. It also takes the scalar step of a
+// device-resident solver loop (BlasTail): a kernel of its own for the sum and
+// another for the step cost 3 to 5 us each, and a copy to the host as much.
 #include "fields.hpp"
 #include "hop_impl.hpp"
 
@@ -254,7 +256,9 @@ __device__ inline void blas_site(const BlasArgs &a, size_t vs, long s, double *r
   }
 }
 
-template <int NR> __device__ inline void block_reduce_store(double *red, double *partials) {
+// SHARED: the partials are read by another block of the same launch
+// (finish_reduction), so they go through to the device's coherence point
+template <int NR, bool SHARED = false> __device__ inline void block_reduce_store(double *red, double *partials) {
   // partials: this launch's (or this right-hand side's) partial array
   __shared__ double lds[kBlasThreads / 64][NR > 0 ? NR : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -269,12 +273,76 @@ template <int NR> __device__ inline void block_reduce_store(double *red, double 
   if (threadIdx.x < NR) {
     double v = 0;
     for (int w = 0; w < (int)(blockDim.x >> 6); w++) v += lds[w][threadIdx.x];
-    partials[blockIdx.x * NR + threadIdx.x] = v;
+    double *o = partials + blockIdx.x * NR + threadIdx.x;
+    if constexpr (SHARED) __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *o = v;
   }
 }
 
+// the scalar steps of the device-resident solver loops, below
+__device__ void blas_tail(const BlasFin &fin, int lane);
+
+// counts this block; true in the last one of the launch. Blocks count in groups
+// of 64 and the groups' last ones at the root, each on a line of its own: one
+// counter for 2048 blocks took 20 us. The counters are left at 0.
+__device__ inline bool counted_last(unsigned *t, unsigned n) {
+  if (n > 1) {
+    if (__hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) return false;
+    __hip_atomic_store(t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  return true;
+}
+__device__ inline bool last_block(unsigned *tickets) {
+  const unsigned n = gridDim.x, group = blockIdx.x / kTicketGroup, groups = (n + kTicketGroup - 1) / kTicketGroup;
+  const unsigned mine = group + 1 < groups ? kTicketGroup : n - group * kTicketGroup;
+  return counted_last(tickets + (group + 1) * kTicketStride, mine) && counted_last(tickets, groups);
+}
+
+// End of a reduction of NR sums: the block's partials, then, in the last block
+// of the launch to get here, their sum in block order (thread t takes blocks
+// t, t + 256, ...) into fin.out and the solver's scalar step. The partials are
+// stored and loaded at agent scope; the wavefront that stored a block's waits
+// for the stores to complete before it counts the block, so the block that
+// reads the full count finds all of them. (An acquire-release increment would
+// order them too, but writes back and invalidates the L2 once per block: 80 us
+// a launch at 2048 blocks.)
+template <int NR> __device__ inline void finish_reduction(double *red, const BlasFin &fin) {
+  block_reduce_store<NR, true>(red, fin.partials);
+  __shared__ double lds[kBlasThreads / 64][NR];
+  __shared__ int last;
+  if (threadIdx.x < 64) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first wavefront's stores
+  if (threadIdx.x == 0) last = last_block(fin.tickets);
+  __syncthreads();
+  if (!last) return;
+#pragma unroll
+  for (int k = 0; k < NR; k++) red[k] = 0;
+  for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x)
+#pragma unroll
+    for (int k = 0; k < NR; k++)
+      red[k] += __hip_atomic_load(fin.partials + b * NR + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    double v = red[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (lane == 0) lds[wave][k] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      double v = 0;
+      for (int w = 0; w < kBlasThreads / 64; w++) v += lds[w][k];
+      fin.out[k] = v;
+    }
+  }
+  if (fin.tail != TAIL_NONE) blas_tail(fin, (int)threadIdx.x);
+}
+
 template <int P, int OP>
-__global__ void __launch_bounds__(kBlasThreads) k_blas(const BlasArgs a0, size_t vs, long vh, double *partials) {
+__global__ void __launch_bounds__(kBlasThreads) k_blas(const BlasArgs a0, size_t vs, long vh, const BlasFin fin) {
   constexpr int NR = nred_of(OP);
   BlasArgs a = a0;
   if (a0.dsc) {
@@ -285,43 +353,18 @@ __global__ void __launch_bounds__(kBlasThreads) k_blas(const BlasArgs a0, size_t
   double red[NR > 0 ? NR : 1] = {0};
   const long stride = (long)gridDim.x * blockDim.x;
   for (long s = (long)blockIdx.x * blockDim.x + threadIdx.x; s < vh; s += stride) blas_site<P, OP>(a, vs, s, red);
-  if constexpr (NR > 0) block_reduce_store<NR>(red, partials);
-}
-
-template <int NR>
-__global__ void __launch_bounds__(kBlasThreads) k_finalize(const double *partials, int nblocks, double *out) {
-  double red[NR];
-#pragma unroll
-  for (int k = 0; k < NR; k++) red[k] = 0;
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
-#pragma unroll
-    for (int k = 0; k < NR; k++) red[k] += partials[b * NR + k];
-  __shared__ double lds[kBlasThreads / 64][NR];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < NR; k++) {
-    double v = red[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) lds[wave][k] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < NR) {
-    double v = 0;
-    for (int w = 0; w < kBlasThreads / 64; w++) v += lds[w][threadIdx.x];
-    out[threadIdx.x] = v;
-  }
+  if constexpr (NR > 0) finish_reduction<NR>(red, fin);
 }
 
 template <int P, int OP>
-static void launch_one(const GeomDesc &g, const BlasArgs &a, double *partials, int nb, hipStream_t st) {
-  k_blas<P, OP><<<nb, kBlasThreads, 0, st>>>(a, g.vs, g.vh, partials);
+static void launch_one(const GeomDesc &g, const BlasArgs &a, const BlasFin &fin, int nb, hipStream_t st) {
+  k_blas<P, OP><<<nb, kBlasThreads, 0, st>>>(a, g.vs, g.vh, fin);
 }
 
 template <int P>
-static hipError_t launch_prec(const GeomDesc &g, int op, const BlasArgs &a, double *partials, int nb, hipStream_t st) {
+static hipError_t launch_prec(const GeomDesc &g, int op, const BlasArgs &a, const BlasFin &fin, int nb, hipStream_t st) {
 #define OPCASE(o) \
-  case o: launch_one<P, o>(g, a, partials, nb, st); break;
+  case o: launch_one<P, o>(g, a, fin, nb, st); break;
   switch (op) {
     OPCASE(B_COPY) OPCASE(B_ZERO) OPCASE(B_AXY) OPCASE(B_AX) OPCASE(B_YPEQX) OPCASE(B_YMEQX)
     OPCASE(B_AYPX) OPCASE(B_AXPY) OPCASE(B_AXPBY) OPCASE(B_NORM2) OPCASE(B_AXPYNORM2) OPCASE(B_XMYNORM2)
@@ -334,16 +377,18 @@ static hipError_t launch_prec(const GeomDesc &g, int op, const BlasArgs &a, doub
   return hipGetLastError();
 }
 
-hipError_t blas_launch(const GeomDesc &g, int op, const BlasArgs &a, double *partials, int *nblocks, hipStream_t st) {
-  long nb = (g.vh + kBlasThreads - 1) / kBlasThreads;
-  if (nb > kMaxBlasBlocks) nb = kMaxBlasBlocks;
-  if (nb < 1) nb = 1;
-  *nblocks = (int)nb;
+static int blas_blocks(const GeomDesc &g) {
+  const long nb = (g.vh + kBlasThreads - 1) / kBlasThreads;
+  return nb > kMaxBlasBlocks ? kMaxBlasBlocks : nb < 1 ? 1 : (int)nb;
+}
+
+hipError_t blas_launch(const GeomDesc &g, int op, const BlasArgs &a, const BlasFin &fin, hipStream_t st) {
+  const int nb = blas_blocks(g);
   switch (g.prec) {
-    case P64: return launch_prec<P64>(g, op, a, partials, (int)nb, st);
-    case P32: return launch_prec<P32>(g, op, a, partials, (int)nb, st);
-    case P16: return launch_prec<P16>(g, op, a, partials, (int)nb, st);
-    case PB16: return launch_prec<PB16>(g, op, a, partials, (int)nb, st);
+    case P64: return launch_prec<P64>(g, op, a, fin, nb, st);
+    case P32: return launch_prec<P32>(g, op, a, fin, nb, st);
+    case P16: return launch_prec<P16>(g, op, a, fin, nb, st);
+    case PB16: return launch_prec<PB16>(g, op, a, fin, nb, st);
   }
   return hipErrorInvalidValue;
 }
@@ -457,36 +502,50 @@ hipError_t mshift_dev_launch(const GeomDesc &g, const MShiftArgs &m, const MsSta
   return hipGetLastError();
 }
 
+// The first wavefront of the block takes these steps, a shift per lane.
 // minvcg.h:279-297 (a, as_s; the counters as the reference counts them)
-__device__ inline void ms_prepare(MsState *ms) {
+__device__ inline void ms_prepare(MsState *ms, int q) {
 #pragma clang fp contract(off)
   const double a = ms->c / ms->cp, b = ms->b;
-  unsigned mask = 0;
-  for (int q = 0; q < ms->nshift; q++)
-    if (!ms->conv[q]) {
-      ms->as[q] = a * ms->zeta[q] * ms->beta[q] / (ms->zeta_prev[q] * b);
-      mask |= 1u << q;
-      ms->site_flops += 72 + 48;
+  const bool open = q < ms->nshift && !ms->conv[q];
+  if (open) ms->as[q] = a * ms->zeta[q] * ms->beta[q] / (ms->zeta_prev[q] * b);
+  const unsigned long long mask = __ballot(open);
+  if (q == 0) {
+    ms->site_flops += (72 + 48) * (unsigned long)__popcll(mask) + 190;
+    ms->a = a;
+    ms->mask_p = (unsigned)mask;
+    ms->do_p0 = 1;
+    ms->cp = ms->c;
+    ms->bp = b;
+  }
+}
+
+// what the host reads: the state of this iteration; a finished solve shows in
+// both entries, since its later iterations skip themselves
+__device__ inline void publish(SolverView *v, int &posts, int done, double progress) {
+  for (int e = 0; e < 2; e++)
+    if (done || e == (posts & 1)) {
+      v[e].done = done;
+      v[e].progress = progress;
     }
-  ms->site_flops += 190;
-  ms->a = a;
-  ms->mask_p = mask;
-  ms->do_p0 = 1;
-  ms->cp = ms->c;
-  ms->bp = b;
+  __threadfence_system();
+  posts++;
 }
 
 __global__ void k_ms_pre(MsState *ms) {
+  const int q = (int)threadIdx.x;
   if (ms->done) {
-    ms->do_p0 = 0;
-    ms->mask_p = 0;
+    if (q == 0) {
+      ms->do_p0 = 0;
+      ms->mask_p = 0;
+    }
     return;
   }
-  ms_prepare(ms);
+  ms_prepare(ms, q);
 }
 
 // minvcg.h:316-320
-__global__ void k_ms_mid(MsState *ms) {
+__device__ inline void ms_mid(MsState *ms) {
 #pragma clang fp contract(off)
   if (ms->done) return;
   double d = 0;
@@ -495,77 +554,77 @@ __global__ void k_ms_mid(MsState *ms) {
   ms->b = -ms->cp / d;
 }
 
-__device__ inline void ms_publish(MsState *ms) {
-  SolverView *v = ms->hview + (ms->posts & 1);
-  v->done = ms->done;
-  v->progress = ms->progress;
-  __threadfence_system();
-  ms->posts++;
-}
-
 // minvcg.h:322-384
-__global__ void k_ms_post(MsState *ms) {
+__device__ inline void ms_post(MsState *ms, int q) {
 #pragma clang fp contract(off)
   if (ms->done) {
     // the x_s updates left pending were applied by this iteration's sweep
-    ms->mask_x = 0;
-    ms->mask_p = 0;
-    ms->do_p0 = 0;
-    ms_publish(ms);
+    if (q == 0) {
+      ms->mask_x = 0;
+      ms->mask_p = 0;
+      ms->do_p0 = 0;
+      publish(ms->hview, ms->posts, ms->done, ms->progress);
+    }
     return;
   }
   double c = 0;
   for (int f = 0; f < ms->nf; f++) c += ms->cf[f];
-  ms->c = c;
   const double a = ms->a, b = ms->b, bp = ms->bp;
-  unsigned pending = 0;
-  bool all = true;
+  const bool mine = q < ms->nshift;
+  const bool open = mine && !ms->conv[q];
   double prog = 0;
-  for (int q = 0; q < ms->nshift; q++) {
-    if (!ms->conv[q]) {
-      const double z0 = ms->zeta[q], z1 = ms->zeta_prev[q];
-      ms->zeta_prev[q] = z0;
-      double z = z0 * z1 * bp;
-      z /= (b * a * (z1 - z0) + z1 * bp * (1.0 - ms->shifts[q] * b));
-      ms->zeta[q] = z;
-      ms->beta[q] = b * z / z0;
-      pending |= 1u << q;
-      const double css = c * z * z;
-      const double ratio = css / ms->rsd_sq[q];
-      if (ratio > prog) prog = ratio;
-      ms->conv[q] = css < ms->rsd_sq[q];
-      if (ms->conv[q]) ms->rsd_sq_final[q] = css;
+  bool conv = mine && !open;
+  if (open) {
+    const double z0 = ms->zeta[q], z1 = ms->zeta_prev[q];
+    ms->zeta_prev[q] = z0;
+    double z = z0 * z1 * bp;
+    z /= (b * a * (z1 - z0) + z1 * bp * (1.0 - ms->shifts[q] * b));
+    ms->zeta[q] = z;
+    ms->beta[q] = b * z / z0;
+    const double css = c * z * z;
+    const double ratio = css / ms->rsd_sq[q];
+    if (ratio > prog) prog = ratio;
+    conv = css < ms->rsd_sq[q];
+    ms->conv[q] = conv;
+    if (conv) ms->rsd_sq_final[q] = css;
+  }
+  const unsigned pending = (unsigned)__ballot(open);
+  const bool all = __ballot(mine && !conv) == 0;
+  for (int off = 32; off > 0; off >>= 1) prog = fmax(prog, __shfl_xor(prog, off, 64));
+  const int k = ms->iters + 1;
+  const bool done = all || k + 1 >= ms->max_iters;
+  if (q == 0) {
+    ms->c = c;
+    ms->mask_x = pending;
+    ms->progress = prog;
+    ms->iters = k;
+    if (all) ms->converged = 1;
+    if (done) {
+      ms->done = 1;
+      ms->mask_p = 0;
+      ms->do_p0 = 0;
     }
-    all = all && ms->conv[q] != 0;
   }
-  ms->mask_x = pending;
-  ms->progress = prog;
-  const int k = ++ms->iters;
-  if (all) {
-    ms->done = 1;
-    ms->converged = 1;
-  } else if (k + 1 >= ms->max_iters) {
-    ms->done = 1;
+  if (!done) {
+    __threadfence_block();  // c of lane 0
+    ms_prepare(ms, q);
   }
-  if (ms->done) {
-    ms->mask_p = 0;
-    ms->do_p0 = 0;
-  } else {
-    ms_prepare(ms);
-  }
-  ms_publish(ms);
+  if (q == 0) publish(ms->hview, ms->posts, done, prog);
 }
 
 hipError_t ms_pre_launch(MsState *st_dev, hipStream_t st) {
-  k_ms_pre<<<1, 1, 0, st>>>(st_dev);
+  k_ms_pre<<<1, 64, 0, st>>>(st_dev);
   return hipGetLastError();
 }
-hipError_t ms_mid_launch(MsState *st_dev, hipStream_t st) {
-  k_ms_mid<<<1, 1, 0, st>>>(st_dev);
-  return hipGetLastError();
+
+// *dst = src, passed as a kernel argument: no staging copy, no wait
+template <typename S> __global__ void k_set_state(S *dst, const S src) {
+  static_assert(sizeof(S) % 8 == 0 && sizeof(S) <= 4000, "a kernel argument of whole double words");
+  const double *s = (const double *)((const char *)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(S *));
+  for (int k = threadIdx.x; k < (int)(sizeof(S) / 8); k += blockDim.x) ((double *)dst)[k] = s[k];
 }
-hipError_t ms_post_launch(MsState *st_dev, hipStream_t st) {
-  k_ms_post<<<1, 1, 0, st>>>(st_dev);
+hipError_t ms_set_launch(MsState *st_dev, const MsState &h, hipStream_t st) {
+  k_set_state<<<1, 64, 0, st>>>(st_dev, h);
   return hipGetLastError();
 }
 
@@ -597,17 +656,8 @@ __device__ inline void bi_freeze(BiState *b, int status, int n_iters) {
   b->done = 1;
   b->pupd[7] = b->supd[7] = b->rxupd[7] = 1.0;
 }
-__device__ inline void bi_publish(BiState *b) {
-  SolverView *v = b->hview + (b->posts & 1);
-  v->done = b->done;
-  v->progress = b->progress;
-  __threadfence_system();
-  b->posts++;
-}
-
-__global__ void k_bi_pre(BiState *b) {
+__device__ inline void bi_pre(BiState *b) {
 #pragma clang fp contract(off)
-  if (b->done) return;
   const int k = b->iters + 1;
   double rho[2] = {0, 0};
   rho[0] += b->ru[1];
@@ -630,7 +680,13 @@ __global__ void k_bi_pre(BiState *b) {
   b->site_flops += 16 * b->sf;
 }
 
-__global__ void k_bi_mid(BiState *b) {
+// a solve that breaks down before its first iteration is published here
+__global__ void k_bi_pre(BiState *b) {
+  bi_pre(b);
+  if (b->done) publish(b->hview, b->posts, 1, b->progress);
+}
+
+__device__ inline void bi_mid(BiState *b) {
 #pragma clang fp contract(off)
   if (b->done) return;
   const int k = b->iters + 1;
@@ -651,7 +707,7 @@ __global__ void k_bi_mid(BiState *b) {
   b->site_flops += 8 * b->sf;
 }
 
-__global__ void k_bi_mid2(BiState *b) {
+__device__ inline void bi_mid2(BiState *b) {
 #pragma clang fp contract(off)
   if (b->done) return;
   const int k = b->iters + 1;
@@ -673,12 +729,9 @@ __global__ void k_bi_mid2(BiState *b) {
   b->rxupd[3] = b->alpha[1];
 }
 
-__global__ void k_bi_post(BiState *b) {
+__device__ inline void bi_post(BiState *b) {
 #pragma clang fp contract(off)
-  if (b->done) {
-    bi_publish(b);
-    return;
-  }
+  if (b->done) return;
   const int k = ++b->iters;
   b->site_flops += 28 * b->sf;
   double r_norm = 0;
@@ -689,24 +742,18 @@ __global__ void k_bi_post(BiState *b) {
     bi_freeze(b, 0, k + 1);
   } else if (k >= b->max_iters) {
     bi_freeze(b, 5 /* QPHIX_ENOCONV */, k + 1);
+  } else {
+    bi_pre(b);
   }
-  bi_publish(b);
+  publish(b->hview, b->posts, b->done, b->progress);
 }
 
 hipError_t bi_pre_launch(BiState *st_dev, hipStream_t st) {
   k_bi_pre<<<1, 1, 0, st>>>(st_dev);
   return hipGetLastError();
 }
-hipError_t bi_mid_launch(BiState *st_dev, hipStream_t st) {
-  k_bi_mid<<<1, 1, 0, st>>>(st_dev);
-  return hipGetLastError();
-}
-hipError_t bi_mid2_launch(BiState *st_dev, hipStream_t st) {
-  k_bi_mid2<<<1, 1, 0, st>>>(st_dev);
-  return hipGetLastError();
-}
-hipError_t bi_post_launch(BiState *st_dev, hipStream_t st) {
-  k_bi_post<<<1, 1, 0, st>>>(st_dev);
+hipError_t bi_set_launch(BiState *st_dev, const BiState &h, hipStream_t st) {
+  k_set_state<<<1, 64, 0, st>>>(st_dev, h);
   return hipGetLastError();
 }
 
@@ -719,7 +766,7 @@ __device__ inline void cgd_freeze(CgDState *c, int status, int n_iters, double r
   c->done = 1;
   c->rmammp[7] = c->aypx[7] = 1.0;
 }
-__global__ void k_cgd_mid(CgDState *c) {
+__device__ inline void cgd_mid(CgDState *c) {
 #pragma clang fp contract(off)
   if (c->done) return;
   c->mv_apps += 2;
@@ -728,7 +775,7 @@ __global__ void k_cgd_mid(CgDState *c) {
   c->site_flops += 4 * c->sf;
   c->rmammp[0] = c->c / d;
 }
-__global__ void k_cgd_post(CgDState *c) {
+__device__ inline void cgd_post(CgDState *c) {
 #pragma clang fp contract(off)
   if (!c->done) {
     double cp = 0;
@@ -749,25 +796,33 @@ __global__ void k_cgd_post(CgDState *c) {
         c->iters = k + 1;
     }
   }
-  SolverView *v = c->hview + (c->posts & 1);
-  v->done = c->done;
-  v->progress = c->progress;
-  __threadfence_system();
-  c->posts++;
+  publish(c->hview, c->posts, c->done, c->progress);
 }
-hipError_t cgd_mid_launch(CgDState *st_dev, hipStream_t st) {
-  k_cgd_mid<<<1, 1, 0, st>>>(st_dev);
+hipError_t cgd_set_launch(CgDState *st_dev, const CgDState &h, hipStream_t st) {
+  k_set_state<<<1, 64, 0, st>>>(st_dev, h);
   return hipGetLastError();
 }
-hipError_t cgd_post_launch(CgDState *st_dev, hipStream_t st) {
-  k_cgd_post<<<1, 1, 0, st>>>(st_dev);
-  return hipGetLastError();
+
+// wave-wide: the first wavefront of the block, after lane 0 wrote the sums
+__device__ void blas_tail(const BlasFin &fin, int lane) {
+  switch (fin.tail) {
+    case TAIL_CG_MID: if (lane == 0) cgd_mid((CgDState *)fin.state); break;
+    case TAIL_CG_POST: if (lane == 0) cgd_post((CgDState *)fin.state); break;
+    case TAIL_BI_MID: if (lane == 0) bi_mid((BiState *)fin.state); break;
+    case TAIL_BI_MID2: if (lane == 0) bi_mid2((BiState *)fin.state); break;
+    case TAIL_BI_POST: if (lane == 0) bi_post((BiState *)fin.state); break;
+    case TAIL_MS_MID: if (lane == 0) ms_mid((MsState *)fin.state); break;
+    case TAIL_MS_POST:
+      __threadfence_block();  // the sums of lane 0
+      ms_post((MsState *)fin.state, lane);
+      break;
+  }
 }
 
 // blas_site<P, B_AXPYNORM2> with the scalar read from device memory
 template <int P>
 __global__ void __launch_bounds__(kBlasThreads) k_axpy_norm2_dev(const double *b, const void *x, void *y, size_t vs,
-                                                                  long vh, double *partials) {
+                                                                  long vh, const BlasFin fin) {
   BlasArgs a;
   a.x = x;
   a.y = nullptr;
@@ -780,23 +835,20 @@ __global__ void __launch_bounds__(kBlasThreads) k_axpy_norm2_dev(const double *b
   double red[1] = {0};
   const long stride = (long)gridDim.x * blockDim.x;
   for (long s = (long)blockIdx.x * blockDim.x + threadIdx.x; s < vh; s += stride) blas_site<P, B_AXPYNORM2>(a, vs, s, red);
-  block_reduce_store<1>(red, partials);
+  finish_reduction<1>(red, fin);
 }
 
-hipError_t axpy_norm2_dev_launch(const GeomDesc &g, const double *b, const void *x, void *y, double *partials,
-                                 double *out, hipStream_t st) {
-  long nb = (g.vh + kBlasThreads - 1) / kBlasThreads;
-  if (nb > kMaxBlasBlocks) nb = kMaxBlasBlocks;
+hipError_t axpy_norm2_dev_launch(const GeomDesc &g, const double *b, const void *x, void *y, const BlasFin &fin,
+                                 hipStream_t st) {
+  const int nb = blas_blocks(g);
   switch (g.prec) {
-    case P64: k_axpy_norm2_dev<P64><<<(int)nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, partials); break;
-    case P32: k_axpy_norm2_dev<P32><<<(int)nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, partials); break;
-    case P16: k_axpy_norm2_dev<P16><<<(int)nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, partials); break;
-    case PB16: k_axpy_norm2_dev<PB16><<<(int)nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, partials); break;
+    case P64: k_axpy_norm2_dev<P64><<<nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, fin); break;
+    case P32: k_axpy_norm2_dev<P32><<<nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, fin); break;
+    case P16: k_axpy_norm2_dev<P16><<<nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, fin); break;
+    case PB16: k_axpy_norm2_dev<PB16><<<nb, kBlasThreads, 0, st>>>(b, x, y, g.vs, g.vh, fin); break;
     default: return hipErrorInvalidValue;
   }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return blas_finalize(partials, (int)nb, 1, out, st);
+  return hipGetLastError();
 }
 
 template <int P, int OP>
@@ -882,16 +934,6 @@ hipError_t blas_multi_launch(const GeomDesc &g, int op, const MultiBlasArgs &m, 
     case 1: k_finalize_multi<1><<<m.n, kBlasThreads, 0, st>>>(partials, (int)nb, out); break;
     case 2: k_finalize_multi<2><<<m.n, kBlasThreads, 0, st>>>(partials, (int)nb, out); break;
     case 3: k_finalize_multi<3><<<m.n, kBlasThreads, 0, st>>>(partials, (int)nb, out); break;
-  }
-  return hipGetLastError();
-}
-
-hipError_t blas_finalize(const double *partials, int nblocks, int nred, double *out, hipStream_t st) {
-  switch (nred) {
-    case 1: k_finalize<1><<<1, kBlasThreads, 0, st>>>(partials, nblocks, out); break;
-    case 2: k_finalize<2><<<1, kBlasThreads, 0, st>>>(partials, nblocks, out); break;
-    case 3: k_finalize<3><<<1, kBlasThreads, 0, st>>>(partials, nblocks, out); break;
-    default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }

@@ -51,11 +51,23 @@ struct BlasArgs {
   const double *dsc;
 };
 int blas_nred(int op);
-// launches op over the geometry; writes nred partial sums per block to
-// partials and returns the number of blocks used
-hipError_t blas_launch(const GeomDesc &g, int op, const BlasArgs &a, double *partials, int *nblocks, hipStream_t st);
-hipError_t blas_finalize(const double *partials, int nblocks, int nred, double *out, hipStream_t st);
+// What the last work-group of a reduction does with the sums: it writes them
+// to out (device or pinned host memory) and takes the scalar step of a
+// device-resident solver loop on `state` (the sums being fields of it)
+enum BlasTail { TAIL_NONE = 0, TAIL_CG_MID, TAIL_CG_POST, TAIL_BI_MID, TAIL_BI_MID2, TAIL_BI_POST, TAIL_MS_MID, TAIL_MS_POST };
+struct BlasFin {
+  double *partials;  // per work-group sums, kMaxBlasBlocks * 3 doubles
+  unsigned *tickets;  // kTickets counters of work-groups done, 0 between launches
+  double *out;
+  int tail;
+  void *state;
+};
+// launches op over the geometry; reductions end in fin (BlasFin), without a
+// further launch
+hipError_t blas_launch(const GeomDesc &g, int op, const BlasArgs &a, const BlasFin &fin, hipStream_t st);
 constexpr int kMaxBlasBlocks = 2048;
+constexpr int kTicketGroup = 64, kTicketStride = 32;  // work-groups per counter, a counter per 128 bytes
+constexpr int kTickets = (1 + kMaxBlasBlocks / kTicketGroup) * kTicketStride;
 
 // Multishift CG vector updates for every shift in one sweep (minvcg.h:298-363):
 //   x_s -= beta_s p_s      for s in mask_x   (uses p_s before its update)
@@ -108,17 +120,15 @@ struct MsState {
 hipError_t mshift_dev_launch(const GeomDesc &g, const MShiftArgs &m, const MsState *st_dev, hipStream_t st);
 // start of the first iteration: a = c / cp, as_s, mask_p, cp = c, bp = b
 hipError_t ms_pre_launch(MsState *st_dev, hipStream_t st);
-// b = -cp / d, d the sum of cf over flavours
-hipError_t ms_mid_launch(MsState *st_dev, hipStream_t st);
-// end of an iteration: c from cf, zeta / beta recurrences, convergence, then
-// the start of the next iteration as ms_pre_launch (or, once the solve is
-// done, only the pending x_s updates for the next sweep)
-hipError_t ms_post_launch(MsState *st_dev, hipStream_t st);
+// TAIL_MS_MID: b = -cp / d, d the sum of cf over flavours.
+// TAIL_MS_POST: end of an iteration, c from cf, zeta / beta recurrences,
+// convergence, then the start of the next iteration as ms_pre_launch (or, once
+// the solve is done, only the pending x_s updates for the next sweep)
 // BiCGStab state in device memory (invbicgstab.h:150-256): the complex
 // scalars, the reductions the device loop writes (<r0, v>, <t, r> with |t|^2,
 // |r|^2 with <r0, r>), and the scalar blocks of the three vector updates
-// (BlasArgs::dsc; [7] = skip once done). Updated by single-thread kernels,
-// so one iteration needs no host round trip.
+// (BlasArgs::dsc; [7] = skip once done). Updated where the reductions end
+// (BlasTail), so one iteration needs no host round trip.
 struct BiState {
   double rho[2], rho_prev[2], alpha[2], omega[2];
   double r0v[2], tr[3], ru[3];
@@ -129,14 +139,15 @@ struct BiState {
   double progress;
   SolverView *hview;
 };
-// start of iteration k: rho = <r0, r>, the breakdown test, beta, p-update scalars
+// start of the first iteration: rho = <r0, r>, the breakdown test, beta,
+// p-update scalars. The tails: TAIL_BI_MID after v = M p and <r0, v>, the
+// breakdown test, alpha, s-update scalars; TAIL_BI_MID2 after t = M r, <t, r>
+// and |t|^2, the breakdown test, omega, x/r-update scalars; TAIL_BI_POST after
+// the x/r update, |r|^2, convergence, the iteration count and the start of the
+// next iteration
 hipError_t bi_pre_launch(BiState *st_dev, hipStream_t st);
-// after v = M p and <r0, v>: the breakdown test, alpha, s-update scalars
-hipError_t bi_mid_launch(BiState *st_dev, hipStream_t st);
-// after t = M r and <t, r>, |t|^2: the breakdown test, omega, x/r-update scalars
-hipError_t bi_mid2_launch(BiState *st_dev, hipStream_t st);
-// after the x/r update: |r|^2, convergence, the iteration count
-hipError_t bi_post_launch(BiState *st_dev, hipStream_t st);
+// *st_dev = h
+hipError_t bi_set_launch(BiState *st_dev, const BiState &h, hipStream_t st);
 
 // CG state in device memory (invcg.h:88-456): c = |r|^2 of the iteration,
 // the reductions |M p|^2 and |r|^2, the scalar blocks of the two vector
@@ -149,15 +160,14 @@ struct CgDState {
   double rsd_sq_final, progress;
   SolverView *hview;
 };
-// after M^+M p and |M p|^2: a = c / d
-hipError_t cgd_mid_launch(CgDState *st_dev, hipStream_t st);
-// after r -= a M^+M p, x += a p, |r|^2: convergence, b = |r|^2 / c
-hipError_t cgd_post_launch(CgDState *st_dev, hipStream_t st);
+// TAIL_CG_MID after M^+M p and |M p|^2: a = c / d. TAIL_CG_POST after
+// r -= a M^+M p, x += a p, |r|^2: convergence, b = |r|^2 / c
+hipError_t cgd_set_launch(CgDState *st_dev, const CgDState &h, hipStream_t st);
+hipError_t ms_set_launch(MsState *st_dev, const MsState &h, hipStream_t st);
 
-// y += (*b) x and |y|^2, the scalar read from device memory; partials as
-// blas_launch, the reduction finalized into *out
-hipError_t axpy_norm2_dev_launch(const GeomDesc &g, const double *b, const void *x, void *y, double *partials,
-                                 double *out, hipStream_t st);
+// y += (*b) x and |y|^2, the scalar read from device memory
+hipError_t axpy_norm2_dev_launch(const GeomDesc &g, const double *b, const void *x, void *y, const BlasFin &fin,
+                                 hipStream_t st);
 
 // one BLAS operation on n right-hand sides in one launch, each with its own
 // operands and first scalar; reductions come back per right-hand side
