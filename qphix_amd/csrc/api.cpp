@@ -1696,7 +1696,7 @@ static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc
 // the device state of a solver's device-resident loop (S: its type)
 template <typename S> static int solver_state(qphix_solver *s, S **st) {
   if (!s->dstate) {
-    const size_t n = std::max(std::max(sizeof(BiState), sizeof(CgDState)), sizeof(MsState));
+    const size_t n = std::max(std::max(sizeof(BiState), sizeof(CgDState)), sizeof(MsState) + kMsDepth * sizeof(MsRec));
     if (hipMalloc(&s->dstate, n) != hipSuccess) {
       (void)hipGetLastError();
       s->dstate = nullptr;
@@ -1715,12 +1715,14 @@ static void clear_view(SolverView *v) {
 }
 
 struct GraphRun {
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  hipGraph_t graph[kMsDepth] = {};
+  hipGraphExec_t exec[kMsDepth] = {};
   hipEvent_t ev[2] = {nullptr, nullptr};
   ~GraphRun() {
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
+    for (int j = 0; j < kMsDepth; j++) {
+      if (exec[j]) (void)hipGraphExecDestroy(exec[j]);
+      if (graph[j]) (void)hipGraphDestroy(graph[j]);
+    }
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
   }
@@ -1732,27 +1734,29 @@ static SolverView *g_bi_view = nullptr;  // pinned host, 2 entries
 // iteration k + 1 before it reads iteration k's view, so the GPU does not wait
 // for the host, except when the residual ratio's trend says k may be the last
 // (or the step limit is near): then it waits for k first. The first iteration
-// runs eagerly (it tunes any kernel not tuned yet); mode 2 captures the second
-// one in a HIP graph and replays it from then on.
-static int device_iterations(int mode, int max_steps, const std::function<int()> &iteration,
-                             SolverView *view) {
+// runs eagerly (it tunes any kernel not tuned yet); mode 2 captures the later
+// ones in HIP graphs and replays them. Iteration k is iteration(k % period): a
+// graph for each.
+static int device_iterations(int mode, int max_steps, const std::function<int(int)> &iteration, SolverView *view,
+                             int period = 1) {
   GraphRun gr;
   HIPCHK(hipEventCreateWithFlags(&gr.ev[0], hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&gr.ev[1], hipEventDisableTiming));
   double prev = -1, prev2 = -1;  // residual ratio of the last two iterations read
   for (int k = 0;; k++) {
-    if (mode == 2 && k == 1) {
+    const int j = k % period;
+    if (mode == 2 && k >= 1 && !gr.exec[j]) {
       HIPCHK(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
-      const int rc = iteration();
-      const hipError_t e = hipStreamEndCapture(g_stream, &gr.graph);
+      const int rc = iteration(j);
+      const hipError_t e = hipStreamEndCapture(g_stream, &gr.graph[j]);
       if (rc) return rc;
       HIPCHK(e);
-      HIPCHK(hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0));
+      HIPCHK(hipGraphInstantiate(&gr.exec[j], gr.graph[j], nullptr, nullptr, 0));
     }
     if (mode == 2 && k >= 1) {
-      HIPCHK(hipGraphLaunch(gr.exec, g_stream));
+      HIPCHK(hipGraphLaunch(gr.exec[j], g_stream));
     } else {
-      TRY(iteration());
+      TRY(iteration(j));
     }
     HIPCHK(hipEventRecord(gr.ev[k & 1], g_stream));
     if (k > 0) {
@@ -1804,7 +1808,7 @@ static int bicgstab_device_loop(qphix_solver *s, void *x, const SV &r0, const SV
     explicit SkipScope(const int *p) { g_hop_skip = p; }
     ~SkipScope() { g_hop_skip = nullptr; }
   } skip_scope(&bs->done);
-  auto iteration = [&]() -> int {
+  auto iteration = [&](int) -> int {
     BlasArgs a = bargs();
     a.x = r[0]; a.y = v[0]; a.o0 = p[0];
     TRY(run_blas_q(g, B_PUPD, a, bs->pupd));
@@ -1864,7 +1868,7 @@ static int cg_device_loop(qphix_solver *s, void *x, const SV &r, const SV &p, SV
     explicit SkipScope(const int *q) { g_hop_skip = q; }
     ~SkipScope() { g_hop_skip = nullptr; }
   } skip_scope(&cs->done);
-  auto iteration = [&]() -> int {
+  auto iteration = [&](int) -> int {
     TRY(op_apply_v(M, mp, cv(p), isign, cb));
     TRY(op_apply_v(M, mmp, cv(mp), -isign, cb));
     BlasArgs a = bargs();
@@ -2744,11 +2748,8 @@ extern "C" int qphix_solve_multi(qphix_solver *s, void *const x[], const void *c
 // from a HIP graph). Once done the state is frozen; a closing sweep applies
 // the x_s updates left pending. Returns 0, -1 (not converged) or a status.
 static SolverView *g_ms_view = nullptr;  // pinned host, 2 entries
-static int device_iterations(int mode, int max_steps, const std::function<int()> &iteration,
-                             SolverView *view);
-
 static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, const double *shifts, int isign, int cb,
-                              const std::vector<void *> &r, const std::vector<void *> &p0,
+                              const std::vector<SV> &ring, const std::vector<void *> &p0,
                               std::vector<void *> &mp, std::vector<void *> &mmp,
                               const std::vector<std::vector<void *>> &p, const std::vector<double> &zeta,
                               const std::vector<double> &zeta_prev, const std::vector<double> &beta,
@@ -2770,6 +2771,8 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
   h.done = s->max_iters <= 1;
   h.site_flops = fl;
   h.hview = g_ms_view;
+  const int depth = (int)ring.size();
+  h.depth = depth;
   for (int q = 0; q < n_shift; q++) {
     h.shifts[q] = shifts[q];
     h.zeta[q] = zeta[q];
@@ -2779,20 +2782,22 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
   }
   MsState *ms;
   TRY(solver_state(s, &ms));
+  h.rec = (MsRec *)(ms + 1);
   clear_view(g_ms_view);
   HIPCHK(ms_set_launch(ms, h, g_stream));
   auto sweep = [&]() -> int {
     for (int f = 0; f < nf; f++) {
-      MShiftArgs m;
+      MsSweep m;
       memset(&m, 0, sizeof(m));
-      m.r = r[f];
+      for (int k = 0; k < depth; k++) m.r[k] = ring[k][f];
       m.p0 = p0[f];
       m.nshift = n_shift;
+      m.depth = depth;
       for (int q = 0; q < n_shift; q++) {
         m.p[q] = p[q][f];
         m.x[q] = x[q * nf + f];
       }
-      HIPCHK(mshift_dev_launch(g->d, m, ms, g_stream));
+      HIPCHK(ms_sweep_launch(g->d, m, ms, g_stream));
     }
     return QPHIX_OK;
   };
@@ -2800,8 +2805,18 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
     explicit SkipScope(const int *p) { g_hop_skip = p; }
     ~SkipScope() { g_hop_skip = nullptr; }
   } skip_scope(&ms->done);
-  auto iteration = [&]() -> int {
-    TRY(sweep());
+  // iteration j of a round: its residual is ring[j], the next one's ring[j + 1].
+  // The shifts' updates are applied in the round's last iteration, before
+  // its residual takes the place of the first.
+  auto iteration = [&](int j) -> int {
+    if (depth > 1) {
+      for (int f = 0; f < nf; f++) {
+        BlasArgs a = bargs();
+        a.x = ring[j][f]; a.o0 = p0[f];
+        TRY(run_blas_q(g, B_AYPX, a, ms->p0upd));
+      }
+    }
+    if (j + 1 == depth) TRY(sweep());
     TRY(op_apply_v(M, mp, (const void *const *)p0.data(), isign, cb));
     TRY(op_apply_v(M, mmp, cv(mp), -isign, cb));
     for (int f = 0; f < nf; f++) {
@@ -2810,13 +2825,13 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
       TRY(run_blas_q(g, B_NORM2, a, nullptr, &ms->cf[f], f + 1 == nf ? TAIL_MS_MID : TAIL_NONE, ms));
     }
     for (int f = 0; f < nf; f++)
-      HIPCHK(axpy_norm2_dev_launch(g->d, &ms->b, mmp[f], r[f],
+      HIPCHK(axpy_norm2_dev_launch(g->d, &ms->b, mmp[f], ring[j][f], ring[(j + 1) % depth][f],
                                    blas_fin(&ms->cf[f], f + 1 == nf ? TAIL_MS_POST : TAIL_NONE, ms), g_stream));
     return QPHIX_OK;
   };
   HIPCHK(ms_pre_launch(ms, g_stream));  // the first iteration's a, as_s
-  TRY(device_iterations(s->ms_mode, s->max_iters, iteration, g_ms_view));
-  TRY(sweep());  // the pending x_s updates (a no-op if the last iteration applied them)
+  TRY(device_iterations(s->ms_mode, s->max_iters, iteration, g_ms_view, depth));
+  TRY(sweep());  // the updates still recorded (a no-op if the last iteration applied them)
   HIPCHK(hipMemcpyAsync(&h, ms, sizeof(h), hipMemcpyDeviceToHost, g_stream));
   HIPCHK(hipStreamSynchronize(g_stream));
   *n_iters = h.iters;
@@ -2867,13 +2882,21 @@ extern "C" int qphix_minvcg_solve(qphix_solver *s, void *const x[], const void *
   const int nf = M->nflav;
   SV r, p0, mp, mmp;
   std::vector<SV> p(n_shift);
-  for (void *w : s->work) qphix_free(w);
-  s->work.clear();
-  TRY(alloc_set(g, nf, r, s));
-  TRY(alloc_set(g, nf, p0, s));
-  TRY(alloc_set(g, nf, mp, s));
-  TRY(alloc_set(g, nf, mmp, s));
-  for (int q = 0; q < n_shift; q++) TRY(alloc_set(g, nf, p[q], s));
+  // work spinors, kept by the solver as those of the other solvers are (they
+  // were allocated, cleared and freed by each solve: 10 of 94 ms at 32^3x64
+  // with 12 shifts)
+  size_t taken = 0;
+  auto take = [&](SV &v) -> int {
+    if (s->work.size() >= (taken + 1) * nf) v.assign(s->work.begin() + taken * nf, s->work.begin() + (taken + 1) * nf);
+    else TRY(alloc_set(g, nf, v, s));
+    taken++;
+    return QPHIX_OK;
+  };
+  TRY(take(r));
+  TRY(take(p0));
+  TRY(take(mp));
+  TRY(take(mmp));
+  for (int q = 0; q < n_shift; q++) TRY(take(p[q]));
   std::vector<double> zeta(n_shift), zeta_prev(n_shift), beta(n_shift), rsd_sq(n_shift);
   std::vector<char> conv(n_shift, 0);
   unsigned long mv = 0, fl = 0;
@@ -2906,10 +2929,20 @@ extern "C" int qphix_minvcg_solve(qphix_solver *s, void *const x[], const void *
   }
   if (s->ms_mode > 0) {
     int kd = 0;
-    const int rc = minvcg_device_loop(s, x, n_shift, shifts, isign, cb, r, p0, mp, mmp, p, zeta, zeta_prev, beta,
+    // room for the residuals of a round of iterations; without it the shifts
+    // are updated in every iteration (as in half storage, which rounds there)
+    std::vector<SV> ring(1, r);
+    if (g->d.prec == P64 || g->d.prec == P32) {
+      const size_t kept = s->work.size();
+      SV v;
+      while (ring.size() < (size_t)kMsDepth && take(v) == QPHIX_OK) ring.push_back(v);
+      if (ring.size() < (size_t)kMsDepth) {
+        ring.resize(1);
+        for (; s->work.size() > kept; s->work.pop_back()) qphix_free(s->work.back());
+      }
+    }
+    const int rc = minvcg_device_loop(s, x, n_shift, shifts, isign, cb, ring, p0, mp, mmp, p, zeta, zeta_prev, beta,
                                       rsd_sq, b, c, cp, fl, rsd_sq_final, n_iters, site_flops, mv_apps, &kd);
-    for (void *w : s->work) qphix_free(w);
-    s->work.clear();
     if (rc < 0) return fail(QPHIX_ENOCONV, "multishift CG did not converge in %d iterations", kd);
     return rc;
   }
@@ -2988,8 +3021,6 @@ extern "C" int qphix_minvcg_solve(qphix_solver *s, void *const x[], const void *
   if (pending_x) TRY(fused(0, 0.0, 0u, pending_x, nullptr));
   if (site_flops) *site_flops = fl;
   if (mv_apps) *mv_apps = mv;
-  for (void *w : s->work) qphix_free(w);
-  s->work.clear();
   return convP ? QPHIX_OK : fail(QPHIX_ENOCONV, "multishift CG did not converge in %d iterations", k);
 }
 

@@ -95,29 +95,47 @@ struct SolverView {
   double progress;
 };
 
+// One iteration's vector updates of the shifted systems, in order:
+// x_s -= beta_s p_s (mask_x), then p_s = zeta_s r + as_s p_s (mask_p)
+struct MsRec {
+  double beta[kMaxShifts], zeta[kMaxShifts], as[kMaxShifts];
+  unsigned mask_x, mask_p;
+};
+// Iterations whose updates of the shifted systems are applied in one sweep
+constexpr int kMsDepth = 8;
 // Multishift CG state in device memory (minvcg.h:279-384): the FP64 scalars
-// and per-shift recurrences of one solve, updated by single-thread kernels
-// between the vector sweeps, so that an iteration needs no host round trip
-// and can be captured in a HIP graph. cf[f] receives per-flavour reductions.
+// and per-shift recurrences of one solve, updated where the reductions end
+// (BlasTail), so that an iteration needs no host round trip and can be
+// captured in a HIP graph. cf[f] receives per-flavour reductions. Iteration k
+// keeps its updates in rec[k % depth].
 struct MsState {
-  double a, b, bp, c, cp, d;
+  double b, bp, c, cp, d;
+  double p0upd[8];  // the p0 update's scalars (BlasArgs::dsc): a, and the skip flag
   double cf[2];
-  double shifts[kMaxShifts], zeta[kMaxShifts], zeta_prev[kMaxShifts], beta[kMaxShifts], as[kMaxShifts];
+  double shifts[kMaxShifts], zeta[kMaxShifts], zeta_prev[kMaxShifts], beta[kMaxShifts];
   double rsd_sq[kMaxShifts], rsd_sq_final[kMaxShifts];
   int conv[kMaxShifts];
-  unsigned mask_x, mask_p;
-  int do_p0, nshift, nf, iters, max_iters, done, converged;
+  int nshift, nf, iters, max_iters, done, converged;
+  int depth, at;  // at: the record of the next sweep
   unsigned long site_flops;
   // largest c zeta_s^2 / target_s over the shifts tested by the last
   // iteration (below 1 for a shift that converged there); lets the host
   // foresee the last iteration
   double progress;
   SolverView *hview;
-  int posts;
+  int posts, pad;
+  MsRec *rec;  // kMsDepth records, right after the state
 };
-// the vector sweep of mshift_launch with a, zeta, as, beta, the masks and
-// do_p0 read from the device state
-hipError_t mshift_dev_launch(const GeomDesc &g, const MShiftArgs &m, const MsState *st_dev, hipStream_t st);
+// the recorded updates of all shifts (m.p, m.x) in one sweep over r[0 .. depth - 1]
+// and, with do_p0, p0 = r[0] + a p0 (depth 1 only)
+struct MsSweep {
+  const void *r[kMsDepth];
+  void *p0;
+  void *p[kMaxShifts];
+  void *x[kMaxShifts];
+  int nshift, depth;
+};
+hipError_t ms_sweep_launch(const GeomDesc &g, const MsSweep &m, const MsState *st_dev, hipStream_t st);
 // start of the first iteration: a = c / cp, as_s, mask_p, cp = c, bp = b
 hipError_t ms_pre_launch(MsState *st_dev, hipStream_t st);
 // TAIL_MS_MID: b = -cp / d, d the sum of cf over flavours.
@@ -165,9 +183,9 @@ struct CgDState {
 hipError_t cgd_set_launch(CgDState *st_dev, const CgDState &h, hipStream_t st);
 hipError_t ms_set_launch(MsState *st_dev, const MsState &h, hipStream_t st);
 
-// y += (*b) x and |y|^2, the scalar read from device memory
-hipError_t axpy_norm2_dev_launch(const GeomDesc &g, const double *b, const void *x, void *y, const BlasFin &fin,
-                                 hipStream_t st);
+// o = y + (*b) x and |o|^2, the scalar read from device memory (o may be y)
+hipError_t axpy_norm2_dev_launch(const GeomDesc &g, const double *b, const void *x, const void *y, void *o,
+                                 const BlasFin &fin, hipStream_t st);
 
 // one BLAS operation on n right-hand sides in one launch, each with its own
 // operands and first scalar; reductions come back per right-hand side
