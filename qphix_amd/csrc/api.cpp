@@ -21,6 +21,7 @@
 #include "blockblas.hpp"
 #include "fields.hpp"
 #include "hop_impl.hpp"
+#include "hop_pair.hpp"
 
 using namespace qphix_amd;
 
@@ -58,7 +59,6 @@ struct qphix_op {
   qphix_dslash d;
   int nflav;
   void *tmp[2];
-  void *tmp2[2];
   std::vector<void *> mtmp;  // per-right-hand-side temporaries of qphix_op_apply_multi
   std::vector<void *> utmp;  // temporaries of the even-odd source preparation / reconstruction
 };
@@ -986,6 +986,64 @@ static HopArgs make_hop_args(const qphix_dslash *d, int cb, const void *u, const
   return a;
 }
 
+// the single-source configuration of a kernel-family member (tuned on its
+// first call, with the operands of t), and its key
+static HopCfg hop_config(const GeomDesc &g, int kind, int isign, const HopArgs &t, std::string &key) {
+  char k[128];
+  snprintf(k, sizeof(k), "p%d c%d k%d s%d %dx%dx%dx%d", g.prec, g.c12, kind, isign, g.L[0], g.L[1], g.L[2], g.L[3]);
+  key = k;
+  auto it = g_tuned.find(key);
+  if (it == g_tuned.end()) {
+    HopCfg c;
+    tune_hop(g, kind, isign, t, c);
+    it = g_tuned.emplace(key, c).first;
+  }
+  return it->second;
+}
+
+// one half of a doublet operator (PairKind) in one launch; the traversal is
+// that of the single-flavour hop it is made of
+static int launch_pair(const qphix_dslash *d, int kind, int isign, int cb, PairArgs &pa, void *const res[2],
+                       const void *const psi[2], const void *const chi[2]) {
+  CHKPTR(pa.a.u);
+  if (isign != 1 && isign != -1) return fail(QPHIX_EDOMAIN, "isign must be +1 or -1, got %d", isign);
+  TRY(check_cb(cb));
+  const bool mix = kind == PD_CLOVER || kind == PD_TM;
+  if ((kind == PD_CLOVER || kind == PA_CLOVER) && !pa.a.clov) return fail(QPHIX_EINVAL, "clover field required");
+  if (kind == PD_CLOVER && (!pa.f[0] || !pa.f[1])) return fail(QPHIX_EINVAL, "full clover fields required");
+  for (int f = 0; f < 2; f++) {
+    if (!res[f] || !psi[f] || (!mix && !chi[f])) return fail(QPHIX_EINVAL, "null spinor of flavour %d", f);
+    pa.a.outs[f] = res[f];
+    pa.a.psis[f] = psi[f];
+    pa.a.chis[f] = mix ? nullptr : chi[f];
+  }
+  const GeomDesc &g = d->g->d;
+  HopArgs t = pa.a;
+  t.psi = psi[0];
+  t.chi = mix ? nullptr : chi[0];
+  std::string key;
+  const HopCfg cfg = hop_config(g, mix ? KD_WILSON : kind == PA_CLOVER ? KA_CLOVER : KA_TM, isign, t, key);
+  pa.a.bz = cfg.bz > 0 ? cfg.bz : 0;
+  pa.a.by = cfg.by;
+  pa.a.slabs = cfg.slabs;
+  hipError_t e;
+  switch (g.prec) {
+    case P64: e = launch_hop_pair_prec<P64>(kind, g.c12 != 0, isign, pa, g_stream); break;
+    case P32: e = launch_hop_pair_prec<P32>(kind, g.c12 != 0, isign, pa, g_stream); break;
+    case P16: e = launch_hop_pair_prec<P16>(kind, g.c12 != 0, isign, pa, g_stream); break;
+    default: e = launch_hop_pair_prec<PB16>(kind, g.c12 != 0, isign, pa, g_stream); break;
+  }
+  if (e != hipSuccess) return fail(QPHIX_EHIP, "doublet hop launch: %s", hipGetErrorString(e));
+  return QPHIX_OK;
+}
+// a result that is also an operand: the flavours then go one after the other
+static bool pair_aliased(void *const res[2], const void *const psi[2], const void *const chi[2]) {
+  for (int f = 0; f < 2; f++)
+    for (int h = 0; h < 2; h++)
+      if (res[f] == psi[h] || res[f] == chi[h]) return true;
+  return res[0] == res[1];
+}
+
 // one kernel-family member applied to n right-hand sides (n = 1: the plain call)
 static int launch_hop_n(const qphix_dslash *d, int kind, int isign, int cb, void *const *res,
                         const void *const *psi, const void *const *chi, int n, const void *u, const void *clov,
@@ -1005,30 +1063,21 @@ static int launch_hop_n(const qphix_dslash *d, int kind, int isign, int cb, void
   const GeomDesc &g = d->g->d;
   HopArgs a = make_hop_args(d, cb, u, clov, coef, alpha, mu, muinv, rho);
   a.dir = dir;
-  char key[128];
-  snprintf(key, sizeof(key), "p%d c%d k%d s%d %dx%dx%dx%d", g.prec, g.c12, kind, isign, g.L[0], g.L[1], g.L[2],
-           g.L[3]);
-  auto it = g_tuned.find(key);
-  if (it == g_tuned.end()) {
-    HopCfg c;
-    HopArgs t = a;
-    t.psi = psi[0];
-    t.chi = needs_chi ? chi[0] : nullptr;
-    tune_hop(g, kind, isign, t, c);
-    it = g_tuned.emplace(key, c).first;
-  }
-  HopCfg cfg = it->second;
+  std::string key;
+  HopArgs t = a;
+  t.psi = psi[0];
+  t.chi = needs_chi ? chi[0] : nullptr;
+  HopCfg cfg = hop_config(g, kind, isign, t, key);
   if (n > 1) {
     // one tuning per power-of-two class of n: solvers that drop converged
     // right-hand sides apply the operator to a shrinking set
     int nb = 2;
     while (nb * 2 <= n && nb < kMaxRhs) nb *= 2;
-    char mkey[160];
-    snprintf(mkey, sizeof(mkey), "%s n%d", key, nb);
+    const std::string mkey = key + " n" + std::to_string(nb);
     auto mt = g_tuned.find(mkey);
     if (mt == g_tuned.end()) {
       HopCfg c = cfg;
-      HopArgs t = a;
+      t = a;
       for (int r = 0; r < n && r < kMaxRhs; r++) {
         t.psis[r] = psi[r];
         t.chis[r] = needs_chi ? chi[r] : nullptr;
@@ -1192,7 +1241,14 @@ extern "C" int qphix_tm_achimbdpsi(qphix_dslash *d, void *res, const void *psi, 
 extern "C" int qphix_tm_two_flav_achimbdpsi(qphix_dslash *d, void *const res[2], const void *const psi[2],
                                             const void *const chi[2], const void *u, double alpha, double beta,
                                             double epsilon, int isign, int cb) {
-  CHKPTR(d); CHKPTR(res); CHKPTR(psi); CHKPTR(chi);
+  ENSURE_INIT();
+  CHKPTR(d); CHKPTR(res); CHKPTR(psi); CHKPTR(chi); CHKPTR(u);
+  if (!pair_aliased(res, psi, chi)) {
+    PairArgs pa{};
+    pa.a = make_hop_args(d, cb, u, nullptr, -beta, alpha, d->p.twisted_mass / (4.0 + d->p.mass), 0, 0);
+    pa.eps = epsilon;
+    return launch_pair(d, PA_TM, isign, cb, pa, res, psi, chi);
+  }
   for (int f = 0; f < 2; f++) {
     TRY(qphix_tm_achimbdpsi(d, res[f], psi[f], chi[f], u, alpha, beta, isign, cb, 1.0 - 2.0 * f));
     TRY(qphix_axpy(d->g, -epsilon, chi[1 - f], res[f]));
@@ -1215,7 +1271,14 @@ extern "C" int qphix_tmclov_achimbdpsi(qphix_dslash *d, void *res, const void *p
 extern "C" int qphix_tmclov_two_flav_achimbdpsi(qphix_dslash *d, void *const res[2], const void *const psi[2],
                                                 const void *const chi[2], const void *u, const void *clov,
                                                 double beta, double epsilon, int isign, int cb) {
-  CHKPTR(d); CHKPTR(res); CHKPTR(psi); CHKPTR(chi);
+  ENSURE_INIT();
+  CHKPTR(d); CHKPTR(res); CHKPTR(psi); CHKPTR(chi); CHKPTR(u);
+  if (!pair_aliased(res, psi, chi)) {
+    PairArgs pa{};
+    pa.a = make_hop_args(d, cb, u, clov, -beta, 0, 0, 0, d->p.prec_mass_rho);
+    pa.eps = epsilon;
+    return launch_pair(d, PA_CLOVER, isign, cb, pa, res, psi, chi);
+  }
   for (int f = 0; f < 2; f++) {
     TRY(qphix_tmclov_achimbdpsi(d, res[f], psi[f], chi[f], u, clov, beta, isign, cb, f));
     TRY(qphix_axpy(d->g, -epsilon, chi[1 - f], res[f]));
@@ -1257,8 +1320,7 @@ extern "C" int qphix_op_create(const qphix_geom *g, const qphix_op_params *p, qp
   op->d.p.prec_mass_rho = (p->kind == QPHIX_OP_NDTMCLOVER) ? p->twisted_mass : p->prec_mass_rho;
   op->nflav = (p->kind == QPHIX_OP_NDTMWILSON || p->kind == QPHIX_OP_NDTMCLOVER) ? 2 : 1;
   for (int f = 0; f < op->nflav; f++) {
-    int r = qphix_alloc_spinor(g, &op->tmp[f]);
-    if (!r && op->nflav == 2) r = qphix_alloc_spinor(g, &op->tmp2[f]);
+    const int r = qphix_alloc_spinor(g, &op->tmp[f]);
     if (r) {
       qphix_op_destroy(op);
       return r;
@@ -1269,10 +1331,7 @@ extern "C" int qphix_op_create(const qphix_geom *g, const qphix_op_params *p, qp
 }
 extern "C" int qphix_op_destroy(qphix_op *op) {
   if (!op) return QPHIX_OK;
-  for (int f = 0; f < 2; f++) {
-    qphix_free(op->tmp[f]);
-    qphix_free(op->tmp2[f]);
-  }
+  for (int f = 0; f < 2; f++) qphix_free(op->tmp[f]);
   for (void *t : op->mtmp) qphix_free(t);
   for (void *t : op->utmp) qphix_free(t);
   delete op;
@@ -1304,15 +1363,22 @@ extern "C" int qphix_op_apply(qphix_op *op, void *const res[], const void *const
     case QPHIX_OP_NDTMWILSON: {
       const double al = 4.0 + p.mass, mu = p.twisted_mass, eps = p.epsilon;
       const double mi = 1.0 / (al * al + mu * mu - eps * eps);
-      for (int f = 0; f < 2; f++) TRY(qphix_wilson_dslash(D, op->tmp[f], in[f], p.u[o], isign, o));
-      const double apimu[2] = {al * mi, -isign * mu * mi};
-      TRY(qphix_two_flav_twisted_mass(op->g, apimu, eps * mi, op->tmp, op->tmp2));
-      return qphix_tm_two_flav_achimbdpsi(D, res, op->tmp2, in, p.u[t], al, 0.25, eps, isign, t);
+      PairArgs pa{};
+      pa.a = make_hop_args(D, o, p.u[o], nullptr, 1.0, 0, 0, 0, 0);
+      pa.t0 = al * mi;
+      pa.t1 = -isign * mu * mi;
+      pa.eps = eps * mi;
+      TRY(launch_pair(D, PD_TM, isign, o, pa, op->tmp, in, nullptr));
+      return qphix_tm_two_flav_achimbdpsi(D, res, (const void *const *)op->tmp, in, p.u[t], al, 0.25, eps, isign, t);
     }
     case QPHIX_OP_NDTMCLOVER: {
-      for (int f = 0; f < 2; f++) TRY(qphix_wilson_dslash(D, op->tmp[f], in[f], p.u[o], isign, o));
-      TRY(qphix_tmclov_two_flav_inverse_clover_term(D, op->tmp2, op->tmp, p.fullclov[o], p.clov_odiag[o], isign));
-      return qphix_tmclov_two_flav_achimbdpsi(D, res, op->tmp2, in, p.u[t], p.clov[t], 0.25, p.epsilon, isign, t);
+      PairArgs pa{};
+      pa.a = make_hop_args(D, o, p.u[o], p.clov_odiag[o], 1.0, 0, 0, 0, 0);
+      pa.f[0] = p.fullclov[o][isign == 1 ? 0 : 1];
+      pa.f[1] = p.fullclov[o][isign == 1 ? 1 : 0];
+      TRY(launch_pair(D, PD_CLOVER, isign, o, pa, op->tmp, in, nullptr));
+      return qphix_tmclov_two_flav_achimbdpsi(D, res, (const void *const *)op->tmp, in, p.u[t], p.clov[t], 0.25,
+                                              p.epsilon, isign, t);
     }
   }
   return fail(QPHIX_EDOMAIN, "unknown operator kind");

@@ -181,7 +181,7 @@ __device__ inline void apply_hop(const cx<T> (&U)[3][3], const cx<T> (&psi)[4][3
   apply_hop_h<MU, S, FWD, C12, FMA>(U, h, coef, tr, ti, acc);
 }
 
-template <int P, bool C12, int ISIGN, int MU>
+template <int P, bool C12, int ISIGN, int MU, bool NT = true>
 __device__ inline void hop_dim(const HopArgs &a, const void *psi_p, long s, long sb, long sf, typename PT<P>::calc cb_coef,
                                typename PT<P>::calc cf_coef, cx<typename PT<P>::calc> (&acc)[4][3]) {
   typedef typename PT<P>::calc T;
@@ -198,7 +198,7 @@ __device__ inline void hop_dim(const HopArgs &a, const void *psi_p, long s, long
     static_assert(!GL::per_link, "FP16 links are read in pairs");
     constexpr int nws = words_of<P>(kSpinorReals);
     T lv[2 * GL::link_reals];
-    load_range<P, GL::nw, MU * GL::pair_words, GL::pair_words, true, false>(a.u, a.vs, s, lv);
+    load_range<P, GL::nw, MU * GL::pair_words, GL::pair_words, NT, false>(a.u, a.vs, s, lv);
     const T su = site_scale<P>(a.u, a.vs, s, GL::nw);
     load_spinor<P, false, false>(psi_p, a.vs, sb, sp);
     const T fb = su * site_scale<P>(psi_p, a.vs, sb, nws);
@@ -214,19 +214,19 @@ __device__ inline void hop_dim(const HopArgs &a, const void *psi_p, long s, long
     T lv[GL::link_reals];
     // backward: U_mu(x-mu)^+ (1 + isign gamma_mu) psi(x-mu)
     load_spinor<P>(psi_p, a.vs, sb, sp);
-    load_range<P, GL::nw, (2 * MU) * GL::link_words, GL::link_words, true>(a.u, a.vs, s, lv);
+    load_range<P, GL::nw, (2 * MU) * GL::link_words, GL::link_words, NT>(a.u, a.vs, s, lv);
     to_spinor(sp, psi);
     make_link<C12>(lv, U);
     apply_hop<MU, ISIGN, false, C12, fma_of<P>()>(U, psi, cb_coef, tr, ti, acc);
     // forward: U_mu(x) (1 - isign gamma_mu) psi(x+mu)
     load_spinor<P>(psi_p, a.vs, sf, sp);
-    load_range<P, GL::nw, (2 * MU + 1) * GL::link_words, GL::link_words, true>(a.u, a.vs, s, lv);
+    load_range<P, GL::nw, (2 * MU + 1) * GL::link_words, GL::link_words, NT>(a.u, a.vs, s, lv);
     to_spinor(sp, psi);
     make_link<C12>(lv, U);
     apply_hop<MU, -ISIGN, true, C12, fma_of<P>()>(U, psi, cf_coef, tr, ti, acc);
   } else {
     T lv[2 * GL::link_reals];
-    load_range<P, GL::nw, MU * GL::pair_words, GL::pair_words, true>(a.u, a.vs, s, lv);
+    load_range<P, GL::nw, MU * GL::pair_words, GL::pair_words, NT>(a.u, a.vs, s, lv);
     load_spinor<P>(psi_p, a.vs, sb, sp);
     to_spinor(sp, psi);
     make_link<C12>(lv, U);
@@ -253,7 +253,7 @@ template <typename T> __device__ inline void shfl_half(const cx<T> (&ho)[2][3], 
     for (int c = 0; c < 3; c++) h[r][c] = mk(__shfl(ho[r][c].r, src, 64), __shfl(ho[r][c].i, src, 64));
 }
 
-template <int P, bool C12, int ISIGN, int MU, bool FWD>
+template <int P, bool C12, int ISIGN, int MU, bool FWD, bool NT>
 __device__ inline void hop_half_shfl(const HopArgs &a, const void *psi_p, const cx<typename PT<P>::calc> (&own)[4][3],
                                      unsigned s, unsigned sn, unsigned s0, bool contig, typename PT<P>::calc coef,
                                      typename PT<P>::calc tr, typename PT<P>::calc ti,
@@ -276,25 +276,26 @@ __device__ inline void hop_half_shfl(const HopArgs &a, const void *psi_p, const 
   cx<T> U[3][3];
   if constexpr (GL::per_link) {
     T lv[GL::link_reals];
-    load_range<P, GL::nw, (2 * MU + (FWD ? 1 : 0)) * GL::link_words, GL::link_words, true>(a.u, a.vs, s, lv);
+    load_range<P, GL::nw, (2 * MU + (FWD ? 1 : 0)) * GL::link_words, GL::link_words, NT>(a.u, a.vs, s, lv);
     make_link<C12>(lv, U);
   } else {
     T lv[2 * GL::link_reals];
-    load_range<P, GL::nw, MU * GL::pair_words, GL::pair_words, true>(a.u, a.vs, s, lv);
+    load_range<P, GL::nw, MU * GL::pair_words, GL::pair_words, NT>(a.u, a.vs, s, lv);
     make_link<C12>(lv + (FWD ? GL::link_reals : 0), U);
   }
   apply_hop_h<MU, S, FWD, C12, fma_of<P>()>(U, h, coef, tr, ti, acc);
 }
 
-template <int P, bool C12, int ISIGN, int MU>
+// NT: links loaded nontemporally (see hop_dim_r)
+template <int P, bool C12, int ISIGN, int MU, bool NT = true>
 __device__ inline void hop_dim_shfl(const HopArgs &a, const void *psi_p, const cx<typename PT<P>::calc> (&own)[4][3],
                                     unsigned s, unsigned sb, unsigned sf, unsigned s0, bool contig,
                                     typename PT<P>::calc coef, cx<typename PT<P>::calc> (&acc)[4][3]) {
   typedef typename PT<P>::calc T;
   const bool tbc = (a.tbc_mask >> MU) & 1;
   const T tr = tbc ? (T)a.tbc_r[MU] : (T)1, ti = tbc ? (T)a.tbc_i[MU] : (T)0;
-  hop_half_shfl<P, C12, ISIGN, MU, false>(a, psi_p, own, s, sb, s0, contig, coef, tr, ti, acc);
-  hop_half_shfl<P, C12, ISIGN, MU, true>(a, psi_p, own, s, sf, s0, contig, coef, tr, ti, acc);
+  hop_half_shfl<P, C12, ISIGN, MU, false, NT>(a, psi_p, own, s, sb, s0, contig, coef, tr, ti, acc);
+  hop_half_shfl<P, C12, ISIGN, MU, true, NT>(a, psi_p, own, s, sf, s0, contig, coef, tr, ti, acc);
 }
 
 // --- clover blocks --------------------------------------------------------
@@ -598,10 +599,11 @@ __device__ inline void full_block_apply_r(const void *fcl, size_t vs, long s, co
 }
 
 // accumulator start of the kernel family: 0, or the A chi part of the
-// achimbdpsi forms, for R right-hand sides at site s
+// achimbdpsi forms, for R right-hand sides at site s (sgn: sign of the
+// twisted mass, -1 for the down flavour of a doublet)
 template <int P, int ISIGN, int KIND, int R, bool NT = true>
 __device__ inline void hop_init_r(const HopArgs &a, unsigned s, const void *const (&chi)[R],
-                                  cx<typename PT<P>::calc> (&acc)[R][4][3]) {
+                                  cx<typename PT<P>::calc> (&acc)[R][4][3], double sgn = 1.0) {
   typedef typename PT<P>::calc T;
   if constexpr (KIND == KA_WILSON || KIND == KA_CLOVER || KIND == KA_TM) {
     cx<T> ch[R][4][3];
@@ -623,7 +625,7 @@ __device__ inline void hop_init_r(const HopArgs &a, unsigned s, const void *cons
       clover_block_apply_r<P, 0, R, false, NT>(a.clov, a.vs, s, ch, acc);
       clover_block_apply_r<P, 1, R, false, NT>(a.clov, a.vs, s, ch, acc);
 #pragma unroll
-      for (int j = 0; j < R; j++) add_ig5((T)(ISIGN * a.rho), ch[j], acc[j]);
+      for (int j = 0; j < R; j++) add_ig5((T)(ISIGN * (sgn * a.rho)), ch[j], acc[j]);
     } else {
       const T al = (T)a.alpha;
 #pragma unroll
@@ -632,7 +634,7 @@ __device__ inline void hop_init_r(const HopArgs &a, unsigned s, const void *cons
         for (int sp = 0; sp < 4; sp++)
 #pragma unroll
           for (int c = 0; c < 3; c++) acc[j][sp][c] = ch[j][sp][c];
-        add_ig5((T)(ISIGN * a.mu), ch[j], acc[j]);
+        add_ig5((T)(ISIGN * (sgn * a.mu)), ch[j], acc[j]);
 #pragma unroll
         for (int sp = 0; sp < 4; sp++)
 #pragma unroll
