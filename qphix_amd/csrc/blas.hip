@@ -725,6 +725,8 @@ __device__ inline void bi_cmul(double *o, const double *a, const double *b) {
   o[0] = re;
   o[1] = im;
 }
+// the end of a solve. Whoever calls this publishes it: the x/r update that
+// carries the publishing step (bi_post) skips itself from here on
 __device__ inline void bi_freeze(BiState *b, int status, int n_iters) {
   b->status = status;
   b->n_iters = n_iters;
@@ -772,6 +774,7 @@ __device__ inline void bi_mid(BiState *b) {
   b->site_flops += 8 * b->sf;
   if (tmp[0] == 0 && tmp[1] == 0) {
     bi_freeze(b, 4, k);
+    publish(b->hview, b->posts, 1, b->progress);
     return;
   }
   bi_cdiv(b->alpha, b->rho, tmp);
@@ -793,6 +796,7 @@ __device__ inline void bi_mid2(BiState *b) {
   const double t_norm = tr[2];
   if (t_norm == 0) {
     bi_freeze(b, 4, k);
+    publish(b->hview, b->posts, 1, b->progress);
     return;
   }
   b->site_flops += 8 * b->sf;
