@@ -830,6 +830,7 @@ static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, 
   HopArgs a = a0;
   a.nrhs = 1;
   a.out = scratch.p;
+  a.skip = nullptr;  // in a solver loop that is over the launches timed here would skip themselves
   for (HopCfg &c : cand) {
     a.bz = c.bz;
     a.slabs = c.slabs;
@@ -864,6 +865,7 @@ static void tune_rhs_tile(const GeomDesc &g, int kind, int isign, const HopArgs 
       return;
     }
   HopArgs a = a0;
+  a.skip = nullptr;  // as in tune_hop
   // ms per source of the rmax sources applied in groups of rt (the last
   // group may be smaller), as launch_hop_n applies them
   auto time_groups = [&](int rt, int reg, int blk) {
