@@ -1719,7 +1719,8 @@ static int solve_cg(qphix_solver *s, void *const *x, const void *const *rhs, dou
     return QPHIX_OK;
   }
   for (int f = 0; f < nf; f++) TRY(qphix_copy_spinor(g, p[f], r[f]));
-  if (s->dev_mode > 0 && nf == 1 && !verbose) return cg_device_loop(s, x[0], r, p, mp, mmp, isign, cb, cp, rsd_sq, sf, st);
+  if (s->dev_mode > 0 && nf == 1 && s->max_iters >= 0 && !verbose)
+    return cg_device_loop(s, x[0], r, p, mp, mmp, isign, cb, cp, rsd_sq, sf, st);
   for (int k = 0; k <= s->max_iters; ++k) {
     const double c = cp;
     TRY(op_apply_v(M, mp, cv(p), isign, cb));
