@@ -438,8 +438,11 @@ int qphix_mr_rxupdate(const qphix_geom *g, void *x, void *r, const void *mr,
  * axpyNorm2 (312), xmyNorm2Spinor (345), innerProduct (520) and
  * innerProductNorm (573) above, with the 1, 1, 1, 2 or 3 results written to
  * d_out (device memory) by kernels on the library stream: no copy, no memset,
- * no synchronisation. Calls share the library's partial-sum buffer, so two of
- * them must not run concurrently on different streams. */
+ * no synchronisation. Each stream, and each capture on a stream, sums in a
+ * buffer of its own (64 of either kind, then the least recently used one goes
+ * to the newcomer), so calls on different streams, and replays of a captured
+ * call beside other reductions and solves, may overlap; replays of one captured
+ * call follow each other. */
 int qphix_norm2_spinor_dev(const qphix_geom *g, const void *x, double *d_out);
 int qphix_axpy_norm2_dev(const qphix_geom *g, double alpha, const void *x, void *y, double *d_out);
 int qphix_xmy_norm2_dev(const qphix_geom *g, void *res, const void *x, const void *y, double *d_out);

@@ -105,8 +105,24 @@ static bool g_init = false;
 static int g_device = 0;
 static hipStream_t g_own_stream = nullptr;
 static hipStream_t g_stream = nullptr;
-static double *g_partials = nullptr;  // device, kMaxBlasBlocks * 3
-static unsigned *g_tickets = nullptr;  // device, the reductions' work-group counters
+// What a reduction sums and counts in (BlasFin): a buffer for each stream, whose
+// launches follow each other, and one for each capture on a stream, whose
+// graph may be replayed beside them. Shared by launches that overlap, the
+// counters would miss their last work-group and stay nonzero for every later
+// launch. Past kReduceBufs streams or captures the least recently used buffer
+// changes hands.
+struct ReduceBuf {
+  double *partials;   // device, kMaxBlasBlocks * 3
+  unsigned *tickets;  // device, kTickets
+  hipStream_t stream;
+  unsigned long long capture, used;  // capture id; use count when last taken (0: never)
+};
+static constexpr int kReduceBufs = 64;
+static ReduceBuf g_reduce[2][kReduceBufs];  // of streams, of captures
+static unsigned long long g_reduce_uses = 0;
+// the buffer of a device-resident solver loop: its launches, eager or captured
+// and replayed, stay on the stream the solve began on
+static ReduceBuf *g_loop_buf = nullptr;
 static double *g_dres = nullptr;      // device, kResults
 static double *g_hres = nullptr;      // pinned host, kResults
 static constexpr int kResults = 4 * kMaxRhs;
@@ -171,9 +187,15 @@ extern "C" int qphix_init(int device) {
   g_device = device;
   HIPCHK(hipStreamCreate(&g_own_stream));
   g_stream = g_own_stream;
-  HIPCHK(hipMalloc(&g_partials, sizeof(double) * kMaxBlasBlocks * 3));
-  HIPCHK(hipMalloc(&g_tickets, sizeof(unsigned) * kTickets));
-  HIPCHK(hipMemset(g_tickets, 0, sizeof(unsigned) * kTickets));
+  {
+    const size_t np = sizeof(double) * kMaxBlasBlocks * 3, nt = sizeof(unsigned) * kTickets;
+    char *pool = nullptr;
+    HIPCHK(hipMalloc(&pool, 2 * kReduceBufs * (np + nt)));
+    HIPCHK(hipMemset(pool, 0, 2 * kReduceBufs * (np + nt)));
+    HIPCHK(hipDeviceSynchronize());
+    for (int k = 0; k < 2 * kReduceBufs; k++, pool += np + nt)
+      g_reduce[k / kReduceBufs][k % kReduceBufs] = ReduceBuf{(double *)pool, (unsigned *)(pool + np), nullptr, 0, 0};
+  }
   HIPCHK(hipMalloc(&g_dres, sizeof(double) * kResults));
   HIPCHK(hipHostMalloc(&g_hres, sizeof(double) * kResults, hipHostMallocDefault));
   HIPCHK(hipEventCreate(&g_ev0));
@@ -455,13 +477,50 @@ extern "C" int qphix_clover_build_noalloc(const qphix_geom *g, const void *u0, c
 // ---------------------------------------------------------------------------
 // BLAS plumbing
 // ---------------------------------------------------------------------------
-static BlasFin blas_fin(double *out, int tail = TAIL_NONE, void *state = nullptr) {
-  return BlasFin{g_partials, g_tickets, out, tail, state};
+// the buffer of the next reduction on g_stream
+static int reduce_buf(ReduceBuf **out) {
+  if (g_loop_buf) {
+    *out = g_loop_buf;
+    return QPHIX_OK;
+  }
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(g_stream, &cs, &id) != hipSuccess) (void)hipGetLastError();
+  const bool captured = cs == hipStreamCaptureStatusActive;
+  if (!captured) id = 0;
+  ReduceBuf *set = g_reduce[captured], *b = nullptr, *oldest = set;
+  for (int k = 0; k < kReduceBufs && !b; k++) {
+    if (set[k].used && set[k].stream == g_stream && set[k].capture == id) b = &set[k];
+    else if (set[k].used < oldest->used) oldest = &set[k];
+  }
+  if (!b) {
+    b = oldest;
+    if (b->used) {
+      // from another stream: its launches end first. From another capture:
+      // counters that an overlap with its graph left nonzero are cleared by
+      // each replay of this one
+      if (!captured) HIPCHK(hipDeviceSynchronize());
+      HIPCHK(blas_clear_tickets(b->tickets, g_stream));
+    }
+    b->stream = g_stream;
+    b->capture = id;
+  }
+  b->used = ++g_reduce_uses;
+  *out = b;
+  return QPHIX_OK;
+}
+static int blas_fin(BlasFin *fin, double *out, int tail = TAIL_NONE, void *state = nullptr) {
+  ReduceBuf *b;
+  TRY(reduce_buf(&b));
+  *fin = BlasFin{b->partials, b->tickets, out, tail, state};
+  return QPHIX_OK;
 }
 // the sums go straight to pinned host memory; the wait is for the kernel alone
 static int run_blas(const qphix_geom *g, int op, const BlasArgs &a, double *out) {
-  HIPCHK(blas_launch(g->d, op, a, blas_fin(g_hres), g_stream));
   const int nr = blas_nred(op);
+  BlasFin fin{};
+  if (nr > 0) TRY(blas_fin(&fin, g_hres));
+  HIPCHK(blas_launch(g->d, op, a, fin, g_stream));
   if (nr > 0) {
     HIPCHK(hipStreamSynchronize(g_stream));
     if (out)
@@ -505,7 +564,9 @@ extern "C" int qphix_stream_calibrate(const qphix_geom *g, int words_in, int wor
 // the reduction left in device memory: kernels only (no copy, no memset, no
 // synchronisation), so the call can be captured in a HIP graph
 static int run_blas_dev(const qphix_geom *g, int op, const BlasArgs &a, double *d_out) {
-  HIPCHK(blas_launch(g->d, op, a, blas_fin(d_out), g_stream));
+  BlasFin fin;
+  TRY(blas_fin(&fin, d_out));
+  HIPCHK(blas_launch(g->d, op, a, fin, g_stream));
   return QPHIX_OK;
 }
 static BlasArgs bargs() {
@@ -1431,7 +1492,9 @@ extern "C" int qphix_op_apply_multi(qphix_op *op, void *const res[], const void 
 
 // n right-hand sides of one BLAS operation in one launch; out gets n * nred values
 static int run_blas_multi(const qphix_geom *g, int op, const MultiBlasArgs &m, double *out) {
-  HIPCHK(blas_multi_launch(g->d, op, m, g_partials, g_dres, g_stream));
+  ReduceBuf *b;
+  TRY(reduce_buf(&b));
+  HIPCHK(blas_multi_launch(g->d, op, m, b->partials, g_dres, g_stream));
   const int nr = blas_nred(op);
   if (nr > 0) {
     HIPCHK(hipMemcpyAsync(g_hres, g_dres, (size_t)m.n * nr * sizeof(double), hipMemcpyDeviceToHost, g_stream));
@@ -1758,7 +1821,9 @@ static int solve_cg(qphix_solver *s, void *const *x, const void *const *rhs, dou
 static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc, double *d_out, int tail,
                       void *state) {
   a.dsc = dsc;
-  HIPCHK(blas_launch(g->d, op, a, blas_fin(d_out, tail, state), g_stream));
+  BlasFin fin{};
+  if (blas_nred(op) > 0) TRY(blas_fin(&fin, d_out, tail, state));
+  HIPCHK(blas_launch(g->d, op, a, fin, g_stream));
   return QPHIX_OK;
 }
 
@@ -1809,6 +1874,12 @@ static SolverView *g_bi_view = nullptr;  // pinned host, 2 entries
 static int device_iterations(int mode, int max_steps, const std::function<int(int)> &iteration, SolverView *view,
                              int period = 1) {
   GraphRun gr;
+  ReduceBuf *buf;
+  TRY(reduce_buf(&buf));
+  struct LoopBuf {
+    explicit LoopBuf(ReduceBuf *b) { g_loop_buf = b; }
+    ~LoopBuf() { g_loop_buf = nullptr; }
+  } loop_buf(buf);
   HIPCHK(hipEventCreateWithFlags(&gr.ev[0], hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&gr.ev[1], hipEventDisableTiming));
   double prev = -1, prev2 = -1;  // residual ratio of the last two iterations read
@@ -2893,9 +2964,11 @@ static int minvcg_device_loop(qphix_solver *s, void *const x[], int n_shift, con
       a.x = mp[f];
       TRY(run_blas_q(g, B_NORM2, a, nullptr, &ms->cf[f], f + 1 == nf ? TAIL_MS_MID : TAIL_NONE, ms));
     }
-    for (int f = 0; f < nf; f++)
-      HIPCHK(axpy_norm2_dev_launch(g->d, &ms->b, mmp[f], ring[j][f], ring[(j + 1) % depth][f],
-                                   blas_fin(&ms->cf[f], f + 1 == nf ? TAIL_MS_POST : TAIL_NONE, ms), g_stream));
+    for (int f = 0; f < nf; f++) {
+      BlasFin fin;
+      TRY(blas_fin(&fin, &ms->cf[f], f + 1 == nf ? TAIL_MS_POST : TAIL_NONE, ms));
+      HIPCHK(axpy_norm2_dev_launch(g->d, &ms->b, mmp[f], ring[j][f], ring[(j + 1) % depth][f], fin, g_stream));
+    }
     return QPHIX_OK;
   };
   HIPCHK(ms_pre_launch(ms, g_stream));  // the first iteration's a, as_s

@@ -377,6 +377,14 @@ static hipError_t launch_prec(const GeomDesc &g, int op, const BlasArgs &a, cons
   return hipGetLastError();
 }
 
+__global__ void k_clear_tickets(unsigned *t) {
+  for (int k = threadIdx.x; k < kTickets; k += blockDim.x) t[k] = 0;
+}
+hipError_t blas_clear_tickets(unsigned *tickets, hipStream_t st) {
+  k_clear_tickets<<<1, kBlasThreads, 0, st>>>(tickets);
+  return hipGetLastError();
+}
+
 static int blas_blocks(const GeomDesc &g) {
   const long nb = (g.vh + kBlasThreads - 1) / kBlasThreads;
   return nb > kMaxBlasBlocks ? kMaxBlasBlocks : nb < 1 ? 1 : (int)nb;

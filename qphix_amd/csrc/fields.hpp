@@ -57,7 +57,8 @@ int blas_nred(int op);
 enum BlasTail { TAIL_NONE = 0, TAIL_CG_MID, TAIL_CG_POST, TAIL_BI_MID, TAIL_BI_MID2, TAIL_BI_POST, TAIL_MS_MID, TAIL_MS_POST };
 struct BlasFin {
   double *partials;  // per work-group sums, kMaxBlasBlocks * 3 doubles
-  unsigned *tickets;  // kTickets counters of work-groups done, 0 between launches
+  unsigned *tickets;  // kTickets counters of work-groups done, 0 between launches;
+                      // not shared with a launch that may overlap this one
   double *out;
   int tail;
   void *state;
@@ -68,6 +69,8 @@ hipError_t blas_launch(const GeomDesc &g, int op, const BlasArgs &a, const BlasF
 constexpr int kMaxBlasBlocks = 2048;
 constexpr int kTicketGroup = 64, kTicketStride = 32;  // work-groups per counter, a counter per 128 bytes
 constexpr int kTickets = (1 + kMaxBlasBlocks / kTicketGroup) * kTicketStride;
+// a kernel, so that it may be captured
+hipError_t blas_clear_tickets(unsigned *tickets, hipStream_t st);
 
 // Multishift CG vector updates for every shift in one sweep (minvcg.h:298-363):
 //   x_s -= beta_s p_s      for s in mask_x   (uses p_s before its update)
