@@ -761,8 +761,9 @@ extern "C" int qphix_dslash_destroy(qphix_dslash *d) {
 // hop-kernel autotuner: per (precision, compression, kernel, isign, lattice) the
 // work-group size and the traversal (natural, or z-block x t tiles per t-slab)
 // are timed once on the first call, into a scratch output so that aliased
-// arguments are never touched twice, and the fastest is kept for the process.
-// All candidates compute bit-identical results; only the order of sites differs.
+// arguments are never touched twice, and the fastest is kept for the process;
+// so is whether the form with a site's terms over wavefronts beats it. All
+// candidates compute bit-identical results; only the order of the work differs.
 // ---------------------------------------------------------------------------
 struct HopCfg {
   int block, bz, slabs;
@@ -771,6 +772,10 @@ struct HopCfg {
   int reg;  // right-hand sides per work-item (register tile; 1 = one per work-item)
   int by;   // rows per traversal tile (0: all of y)
   int lds;  // dynamic LDS bytes per work-group capping the work-groups per CU (0: none)
+  // one source: HopArgs::split. The traversal stays that of the best form with a
+  // work-item per site, for the launches that have no other (several sources,
+  // doublets); ms is the split form's time where it is the faster
+  int split;
 };
 static std::map<std::string, HopCfg> g_tuned;
 static int g_tune_enabled = -1;            // -1: read QPHIX_TUNE on first use
@@ -882,7 +887,6 @@ static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, 
         if (bz <= g.L[2] && g.L[2] % bz == 0 && g.L[3] % sl == 0 && g.L[3] / sl >= 2)
           cand.push_back({blk, bz, sl, 0, 1, 1});
   }
-  if (kind != KD_DIR) cand.push_back({256, -1, 1, 0, 1, 1});  // the eight terms over wavefronts
   DevBuf scratch;
   if (hipMalloc(&scratch.p, spinor_bytes(g)) != hipSuccess) {
     (void)hipGetLastError();
@@ -898,6 +902,15 @@ static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, 
     c.ms = time_hop(g, kind, isign, a, c.block, 4);
     if (best.ms < 0 || c.ms < best.ms) best = c;
   }
+  if (kind == KD_DIR) return;
+  a.bz = 0;
+  a.slabs = 1;
+  a.split = 1;
+  const double ms = time_hop(g, kind, isign, a, 256, 4);
+  if (ms < best.ms) {
+    best.split = 1;
+    best.ms = ms;
+  }
 }
 
 // right-hand-side tiling for n right-hand sides, given the single-RHS
@@ -908,6 +921,7 @@ static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, 
 static void tune_rhs_tile(const GeomDesc &g, int kind, int isign, const HopArgs &a0, int n, HopCfg &cfg) {
   cfg.rt = n < kMaxRhs ? n : kMaxRhs;
   cfg.reg = 1;
+  if (cfg.split > 0) cfg.split = 0;  // a form for one source
   if (g_forced_reg > 0) {
     cfg.reg = g_forced_reg;
     cfg.rt = g_forced_rt;
@@ -961,7 +975,6 @@ static void tune_rhs_tile(const GeomDesc &g, int kind, int isign, const HopArgs 
   // first the tiling under the single-RHS traversal; the matrix-core form
   // (reg 8) is not a candidate: it runs slower per source than the register
   // tiles (qphix_tune_rhs(8, n) still forces it)
-  if (cfg.bz < 0) cfg.bz = 0;  // a register tile has no split form
   a.bz = cfg.bz;
   a.slabs = cfg.slabs;
   std::vector<HopCfg> tiles;
@@ -1086,7 +1099,7 @@ static int launch_pair(const qphix_dslash *d, int kind, int isign, int cb, PairA
   t.chi = mix ? nullptr : chi[0];
   std::string key;
   const HopCfg cfg = hop_config(g, mix ? KD_WILSON : kind == PA_CLOVER ? KA_CLOVER : KA_TM, isign, t, key);
-  pa.a.bz = cfg.bz > 0 ? cfg.bz : 0;
+  pa.a.bz = cfg.bz;
   pa.a.by = cfg.by;
   pa.a.slabs = cfg.slabs;
   hipError_t e;
@@ -1154,6 +1167,11 @@ static int launch_hop_n(const qphix_dslash *d, int kind, int isign, int cb, void
   a.slabs = cfg.slabs;
   a.by = cfg.by;
   a.lds_cap = cfg.lds;
+  if (n == 1 && cfg.split > 0) {
+    a.split = 1;
+    a.bz = a.by = a.lds_cap = 0;
+    a.slabs = 1;
+  }
   const int rt = n == 1 ? 1 : (cfg.rt > 0 ? cfg.rt : 1);
   const int reg = n == 1 ? 1 : cfg.reg;
   for (int r0 = 0; r0 < n; r0 += rt) {
@@ -1224,9 +1242,9 @@ extern "C" const char *qphix_tune_summary(void) {
   out.clear();
   for (auto &kv : g_tuned) {
     char line[256];
-    snprintf(line, sizeof(line), "%s: block %d bz %d by %d slabs %d rhs-tile %d reg-tile %d lds %d %.4f ms\n",
+    snprintf(line, sizeof(line), "%s: block %d bz %d by %d slabs %d rhs-tile %d reg-tile %d lds %d %s%.4f ms\n",
              kv.first.c_str(), kv.second.block, kv.second.bz, kv.second.by, kv.second.slabs, kv.second.rt,
-             kv.second.reg, kv.second.lds, kv.second.ms);
+             kv.second.reg, kv.second.lds, kv.second.split > 0 ? "split " : "", kv.second.ms);
     out += line;
   }
   return out.c_str();

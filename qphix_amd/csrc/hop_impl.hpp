@@ -39,12 +39,14 @@ struct HopArgs {
   double tbc_r[4], tbc_i[4];
   int tbc_mask;
   double alpha, mu, muinv, rho;
-  // traversal: bz = 0 is the natural site order, bz < 0 too, with the eight
-  // terms of a site split over wavefronts (hop_split.hpp); otherwise the (y, z) cross
+  // traversal: bz = 0 is the natural site order; otherwise the (y, z) cross
   // section is cut into tiles of by rows (by = 0: all of y) by bz planes and
   // each of `slabs` t-slabs is walked tile by tile, t innermost, so consecutive
   // work-groups of one XCD reuse the source spinor slices they share
   int bz, slabs, by;
+  // the eight terms of a site over wavefronts (hop_split.hpp, natural order):
+  // 1: the tuner's choice, 0: by rule
+  int split;
   int dir;  // KD_DIR only
   // multi-RHS: nrhs > 1 applies the operator to psis[r] -> outs[r] (chis[r]);
   // the right-hand side is the fastest index of the work-group order, so the
