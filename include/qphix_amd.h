@@ -68,7 +68,10 @@ int qphix_timer_stop(double *ms);
 /* Tuning hooks (no reference counterpart: the reference's blocking
  * parameters By/Bz/Sy/Sz play this role on the CPU). Hop kernels are
  * autotuned on first use per lattice unless QPHIX_TUNE=0; block is the
- * default work-group size (64..256, multiple of 64) when tuning is off. */
+ * default work-group size (64..256, multiple of 64) when tuning is off or the
+ * lattice too small to be tuned (below 2^17 sites of a parity). Small lattices
+ * otherwise take a form with a site's hop terms over several wavefronts, unless
+ * a work-group size or configuration was asked for. */
 int qphix_set_hop_block(int block);
 /* mode 0: no tuning; 1: autotune on first use; 2: force (block, bz, slabs):
  * bz z-planes per tile, slabs t-slabs (bz = 0: natural site order) */

@@ -128,6 +128,7 @@ static double *g_hres = nullptr;      // pinned host, kResults
 static constexpr int kResults = 4 * kMaxRhs;
 static hipEvent_t g_ev0, g_ev1;
 static int g_hop_block = 256;
+static bool g_hop_block_set = false;  // by qphix_set_hop_block
 
 static int fail(int code, const char *fmt, ...) {
   char buf[512];
@@ -234,6 +235,7 @@ extern "C" int qphix_timer_stop(double *ms) {
 extern "C" int qphix_set_hop_block(int b) {
   if (b <= 0 || b > 256 || (b & 63)) return fail(QPHIX_EDOMAIN, "hop block %d must be 64, 128, 192 or 256", b);
   g_hop_block = b;
+  g_hop_block_set = true;
   return QPHIX_OK;
 }
 
@@ -869,8 +871,10 @@ static double time_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a,
 
 static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, HopCfg &best) {
   best = HopCfg{g_hop_block, 0, 1, -1, 1, 1};
+  if (g_hop_block_set) best.split = -1;  // an untuned launch has the caller's work-group size
   if (g_forced.block > 0) {
     best = g_forced;
+    best.split = -1;
     if (best.bz > 0 && (g.L[2] % best.bz || g.L[3] % best.slabs)) {
       best.bz = 0;
       best.slabs = 1;
@@ -1167,8 +1171,8 @@ static int launch_hop_n(const qphix_dslash *d, int kind, int isign, int cb, void
   a.slabs = cfg.slabs;
   a.by = cfg.by;
   a.lds_cap = cfg.lds;
-  if (n == 1 && cfg.split > 0) {
-    a.split = 1;
+  a.split = cfg.split;
+  if (cfg.split > 0) {  // one source
     a.bz = a.by = a.lds_cap = 0;
     a.slabs = 1;
   }

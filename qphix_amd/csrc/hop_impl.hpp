@@ -45,7 +45,7 @@ struct HopArgs {
   // work-groups of one XCD reuse the source spinor slices they share
   int bz, slabs, by;
   // the eight terms of a site over wavefronts (hop_split.hpp, natural order):
-  // 1: the tuner's choice, 0: by rule
+  // 1: the tuner's choice, 0: by rule, -1: no, the caller fixed the launch
   int split;
   int dir;  // KD_DIR only
   // multi-RHS: nrhs > 1 applies the operator to psis[r] -> outs[r] (chis[r]);

@@ -39,8 +39,8 @@ constexpr long split_sites(int p, int kind) {
   return p == P64 ? 49152 : p == P32 ? (kind == KD_FULL ? 49152 : (1l << 17) - 1) : 45056;
 }
 inline bool use_split(int p, int kind, const HopArgs &a, int nr) {
-  if (kind == KD_DIR || a.bz != 0) return false;
-  return a.split > 0 || (a.lds_cap == 0 && (long)a.vh * nr <= split_sites(p, kind));
+  if (kind == KD_DIR || a.bz != 0 || a.split < 0) return false;
+  return a.split > 0 || (long)a.vh * nr <= split_sites(p, kind);
 }
 
 // one term: lds[k * 64 + lane] gets the 12 reals of coef U h
