@@ -364,7 +364,12 @@ int qphix_minvcg_set_mode(qphix_solver *s, int mode);
  * and silent solves (the others run mode 0); all three give bit-identical
  * solutions, counters and statuses. */
 int qphix_solver_set_mode(qphix_solver *s, int mode);
-/* x[shift * nflav + f]; rsd_sq_final[n_shift] */
+/* x[shift * nflav + f]; rsd_sq_final[n_shift]. The solver keeps its work spinors
+ * for the next solve: n_shift + 4, and with modes 1 and 2 in FP64 and FP32 seven
+ * more where memory allows, times the flavours (4.6 GB at 32^3x64 FP64 with 12
+ * shifts). They are freed by qphix_solver_destroy, by an allocation of this
+ * library that would fail without them, and at the end of a solve after which
+ * all multishift solvers would keep more than an eighth of the device's memory. */
 int qphix_minvcg_solve(qphix_solver *s, void *const x[], const void *const rhs[],
                        int n_shift, const double *shifts, const double *rsd_target,
                        int isign, int verbose, int target_cb, int *n_iters,

@@ -68,6 +68,7 @@ struct qphix_solver {
   qphix_op *M;
   int max_iters;
   std::vector<void *> work;  // solver-owned spinors
+  size_t work_bytes = 0;     // what an idle multishift solver keeps of them
   // Richardson
   qphix_solver *inner;
   double delta;
@@ -127,6 +128,7 @@ static double *g_dres = nullptr;      // device, kResults
 static double *g_hres = nullptr;      // pinned host, kResults
 static constexpr int kResults = 4 * kMaxRhs;
 static hipEvent_t g_ev0, g_ev1;
+static size_t g_memory = 0;  // bytes of the device
 static int g_hop_block = 256;
 static bool g_hop_block_set = false;  // by qphix_set_hop_block
 
@@ -186,6 +188,7 @@ extern "C" int qphix_init(int device) {
   if (device < 0 || device >= n) return fail(QPHIX_EDOMAIN, "device %d out of range (%d devices)", device, n);
   HIPCHK(hipSetDevice(device));
   g_device = device;
+  HIPCHK(hipDeviceTotalMem(&g_memory, device));
   HIPCHK(hipStreamCreate(&g_own_stream));
   g_stream = g_own_stream;
   {
@@ -293,11 +296,21 @@ extern "C" int qphix_geom_info(const qphix_geom *g, int latt[4], int *prec, int 
   return QPHIX_OK;
 }
 
+static bool release_idle_work();
+// hipMalloc; when memory is out, again without what idle solvers keep
+template <typename T> static hipError_t dev_malloc(T **p, size_t n) {
+  hipError_t e = hipMalloc(p, n);
+  if (e == hipErrorOutOfMemory && release_idle_work()) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, n);
+  }
+  return e;
+}
 static int alloc_zeroed(size_t n, void **p) {
   ENSURE_INIT();
   CHKPTR(p);
   void *q = nullptr;
-  if (hipMalloc(&q, n) != hipSuccess) {
+  if (dev_malloc(&q, n) != hipSuccess) {
     (void)hipGetLastError();
     return fail(QPHIX_ENOMEM, "hipMalloc of %zu bytes failed", n);
   }
@@ -318,6 +331,41 @@ extern "C" int qphix_free(void *p) {
   return QPHIX_OK;
 }
 
+// Work spinors that multishift solvers keep from one solve to the next: of all
+// solvers together at most an eighth of the device's memory (a solve that
+// would keep more frees its own at its end), and none of an idle solver once an
+// allocation of the library fails.
+static std::vector<qphix_solver *> g_keepers;     // multishift solvers with work spinors
+static qphix_solver *g_keeper_busy = nullptr;     // the one in its solve
+static void release_work(qphix_solver *s) {
+  for (void *w : s->work) qphix_free(w);
+  s->work.clear();
+  s->work_bytes = 0;
+  g_keepers.erase(std::remove(g_keepers.begin(), g_keepers.end(), s), g_keepers.end());
+}
+static bool release_idle_work() {
+  const std::vector<qphix_solver *> all = g_keepers;
+  bool any = false;
+  for (qphix_solver *s : all)
+    if (s != g_keeper_busy) {
+      release_work(s);
+      any = true;
+    }
+  return any;
+}
+struct KeepWork {  // for the length of a multishift solve
+  qphix_solver *s;
+  explicit KeepWork(qphix_solver *x) : s(x) { g_keeper_busy = s; }
+  ~KeepWork() {
+    g_keeper_busy = nullptr;
+    s->work_bytes = s->work.size() * s->M->g->bytes[0];
+    if (std::find(g_keepers.begin(), g_keepers.end(), s) == g_keepers.end()) g_keepers.push_back(s);
+    size_t all = 0;
+    for (const qphix_solver *k : g_keepers) all += k->work_bytes;
+    if (all > g_memory / 8) release_work(s);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // packers, generation, conversion, clover build
 // ---------------------------------------------------------------------------
@@ -329,7 +377,7 @@ struct DevBuf {
 };
 
 static int stage_in(DevBuf &b, const double *src, size_t n) {
-  if (hipMalloc(&b.p, n * sizeof(double)) != hipSuccess) {
+  if (dev_malloc(&b.p, n * sizeof(double)) != hipSuccess) {
     (void)hipGetLastError();
     return fail(QPHIX_ENOMEM, "staging allocation of %zu doubles failed", n);
   }
@@ -354,7 +402,7 @@ extern "C" int qphix_unpack_spinor(const qphix_geom *g, double *dst, const void 
   TRY(check_cb(cb));
   DevBuf b;
   const size_t n = (size_t)g->d.vh * kSpinorReals;
-  if (hipMalloc(&b.p, n * sizeof(double)) != hipSuccess) return fail(QPHIX_ENOMEM, "staging allocation failed");
+  if (dev_malloc(&b.p, n * sizeof(double)) != hipSuccess) return fail(QPHIX_ENOMEM, "staging allocation failed");
   HIPCHK(fld_unpack_spinor(g->d, (double *)b.p, src, g_stream));
   HIPCHK(hipMemcpyAsync(dst, b.p, n * sizeof(double), hipMemcpyDeviceToHost, g_stream));
   HIPCHK(hipStreamSynchronize(g_stream));
@@ -386,7 +434,7 @@ extern "C" int qphix_unpack_clover(const qphix_geom *g, double *dst, const void 
   TRY(check_cb(cb));
   DevBuf b;
   const size_t n = (size_t)g->d.vh * kCloverReals;
-  if (hipMalloc(&b.p, n * sizeof(double)) != hipSuccess) return fail(QPHIX_ENOMEM, "staging allocation failed");
+  if (dev_malloc(&b.p, n * sizeof(double)) != hipSuccess) return fail(QPHIX_ENOMEM, "staging allocation failed");
   HIPCHK(fld_unpack_clover(g->d, (double *)b.p, src, g_stream));
   HIPCHK(hipMemcpyAsync(dst, b.p, n * sizeof(double), hipMemcpyDeviceToHost, g_stream));
   HIPCHK(hipStreamSynchronize(g_stream));
@@ -435,7 +483,7 @@ extern "C" int qphix_gen_gauge(const qphix_geom *g, void *u0, void *u1, uint64_t
   CHKPTR(g); CHKPTR(u0); CHKPTR(u1);
   DevBuf b;
   const size_t n = (size_t)g->d.vh * 2 * 72;
-  if (hipMalloc(&b.p, n * sizeof(double)) != hipSuccess) {
+  if (dev_malloc(&b.p, n * sizeof(double)) != hipSuccess) {
     (void)hipGetLastError();
     return fail(QPHIX_ENOMEM, "gauge staging allocation failed");
   }
@@ -892,7 +940,7 @@ static void tune_hop(const GeomDesc &g, int kind, int isign, const HopArgs &a0, 
           cand.push_back({blk, bz, sl, 0, 1, 1});
   }
   DevBuf scratch;
-  if (hipMalloc(&scratch.p, spinor_bytes(g)) != hipSuccess) {
+  if (dev_malloc(&scratch.p, spinor_bytes(g)) != hipSuccess) {
     (void)hipGetLastError();
     return;  // keep the default configuration
   }
@@ -939,7 +987,7 @@ static void tune_rhs_tile(const GeomDesc &g, int kind, int isign, const HopArgs 
   const int rmax = cfg.rt;
   std::vector<DevBuf> outs(rmax);
   for (int r = 0; r < rmax; r++)
-    if (hipMalloc(&outs[r].p, spinor_bytes(g)) != hipSuccess) {
+    if (dev_malloc(&outs[r].p, spinor_bytes(g)) != hipSuccess) {
       (void)hipGetLastError();
       return;
     }
@@ -1736,7 +1784,7 @@ extern "C" int qphix_minvcg_create(qphix_op *M, int max_iters, int max_shifts, q
 }
 extern "C" int qphix_solver_destroy(qphix_solver *s) {
   if (!s) return QPHIX_OK;
-  for (void *p : s->work) qphix_free(p);
+  release_work(s);
   for (void *p : s->mwork) qphix_free(p);
   qphix_free(s->dstate);
   delete s;
@@ -1853,7 +1901,7 @@ static int run_blas_q(const qphix_geom *g, int op, BlasArgs a, const double *dsc
 template <typename S> static int solver_state(qphix_solver *s, S **st) {
   if (!s->dstate) {
     const size_t n = std::max(std::max(sizeof(BiState), sizeof(CgDState)), sizeof(MsState) + kMsDepth * sizeof(MsRec));
-    if (hipMalloc(&s->dstate, n) != hipSuccess) {
+    if (dev_malloc(&s->dstate, n) != hipSuccess) {
       (void)hipGetLastError();
       s->dstate = nullptr;
       return fail(QPHIX_ENOMEM, "solver state allocation");
@@ -2588,10 +2636,10 @@ constexpr size_t kMatDoubles = (size_t)kMaxRhs * kMaxRhs * 2;
 
 static int block_buffers() {
   if (g_gram_part) return QPHIX_OK;
-  HIPCHK(hipMalloc(&g_gram_part, kGramPartials * sizeof(double)));
-  HIPCHK(hipMalloc(&g_gram_dev, kMatDoubles * sizeof(double)));
+  HIPCHK(dev_malloc(&g_gram_part, kGramPartials * sizeof(double)));
+  HIPCHK(dev_malloc(&g_gram_dev, kMatDoubles * sizeof(double)));
   HIPCHK(hipHostMalloc(&g_gram_host, kMatDoubles * sizeof(double), hipHostMallocDefault));
-  HIPCHK(hipMalloc(&g_mat_dev, 4 * kMatDoubles * sizeof(double)));
+  HIPCHK(dev_malloc(&g_mat_dev, 4 * kMatDoubles * sizeof(double)));
   HIPCHK(hipHostMalloc(&g_mat_host, 4 * kMatDoubles * sizeof(double), hipHostMallocDefault));
   return QPHIX_OK;
 }
@@ -3046,9 +3094,9 @@ extern "C" int qphix_minvcg_solve(qphix_solver *s, void *const x[], const void *
   const int nf = M->nflav;
   SV r, p0, mp, mmp;
   std::vector<SV> p(n_shift);
-  // work spinors, kept by the solver as those of the other solvers are (they
-  // were allocated, cleared and freed by each solve: 10 of 94 ms at 32^3x64
-  // with 12 shifts)
+  // work spinors, kept by the solver (KeepWork: allocated, cleared and freed by
+  // each solve they took 10 of 94 ms at 32^3x64 with 12 shifts)
+  const KeepWork keep(s);
   size_t taken = 0;
   auto take = [&](SV &v) -> int {
     if (s->work.size() >= (taken + 1) * nf) v.assign(s->work.begin() + taken * nf, s->work.begin() + (taken + 1) * nf);
@@ -3290,18 +3338,18 @@ extern "C" int qphix_batch_create(qphix_op *const ops[], int nsys, qphix_batch *
       v->push_back(q);
     }
   const size_t nn = nsys;
-  bool ok = hipMalloc(&b->d_off, sizeof(int) * (nn + 1)) == hipSuccess &&
-            hipMalloc(&b->d_active, sizeof(int) * nn) == hipSuccess &&
-            hipMalloc(&b->d_hop, sizeof(HopSeg) * 4 * nn) == hipSuccess &&
-            hipMalloc(&b->d_seg, sizeof(SegVec) * 8 * nn) == hipSuccess &&
-            hipMalloc(&b->d_state, sizeof(CgState) * nn) == hipSuccess &&
-            hipMalloc(&b->d_alpha, sizeof(double) * nn) == hipSuccess &&
-            hipMalloc(&b->d_beta, sizeof(double) * nn) == hipSuccess &&
-            hipMalloc(&b->d_d, sizeof(double) * nn) == hipSuccess &&
-            hipMalloc(&b->d_cp, sizeof(double) * nn) == hipSuccess &&
-            hipMalloc(&b->d_rsd, sizeof(double) * nn) == hipSuccess &&
-            hipMalloc(&b->d_partials, sizeof(double) * (size_t)b->off[nsys]) == hipSuccess &&
-            hipMalloc(&b->d_hoff, sizeof(int) * (size_t)(b->nhseg + 1)) == hipSuccess;
+  bool ok = dev_malloc(&b->d_off, sizeof(int) * (nn + 1)) == hipSuccess &&
+            dev_malloc(&b->d_active, sizeof(int) * nn) == hipSuccess &&
+            dev_malloc(&b->d_hop, sizeof(HopSeg) * 4 * nn) == hipSuccess &&
+            dev_malloc(&b->d_seg, sizeof(SegVec) * 8 * nn) == hipSuccess &&
+            dev_malloc(&b->d_state, sizeof(CgState) * nn) == hipSuccess &&
+            dev_malloc(&b->d_alpha, sizeof(double) * nn) == hipSuccess &&
+            dev_malloc(&b->d_beta, sizeof(double) * nn) == hipSuccess &&
+            dev_malloc(&b->d_d, sizeof(double) * nn) == hipSuccess &&
+            dev_malloc(&b->d_cp, sizeof(double) * nn) == hipSuccess &&
+            dev_malloc(&b->d_rsd, sizeof(double) * nn) == hipSuccess &&
+            dev_malloc(&b->d_partials, sizeof(double) * (size_t)b->off[nsys]) == hipSuccess &&
+            dev_malloc(&b->d_hoff, sizeof(int) * (size_t)(b->nhseg + 1)) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
     qphix_batch_destroy(b);
