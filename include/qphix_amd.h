@@ -352,10 +352,11 @@ int qphix_solve_multi(qphix_solver *s, void *const x[], const void *const rhs[],
 /* How qphix_minvcg_solve runs its iterations (no reference counterpart; the
  * reference keeps the recurrences on the host, minvcg.h:279-384). mode 0: FP64
  * scalars and the zeta / beta recurrences on the host, one host round trip per
- * iteration; 1: all of them in device memory, updated by device kernels
- * between the vector sweeps, no host round trip; 2 (the default): as 1, with
- * one iteration captured in a HIP graph and replayed. All three give
- * bit-identical solutions and counters. */
+ * iteration; 1 (the default): all of them in device memory, updated where the
+ * reductions end, no host round trip; 2: as 1, with the iterations captured in
+ * HIP graphs (FP64 and FP32: one for each of the eight iterations between two
+ * sweeps over the shifts) and replayed. All three give bit-identical solutions
+ * and counters. */
 int qphix_minvcg_set_mode(qphix_solver *s, int mode);
 /* The same control for CG and BiCGStab solvers (no reference counterpart;
  * the reference keeps their scalars on the host, invcg.h:293-343,

@@ -497,8 +497,8 @@ def InvRichardsonMultiPrec(M_outer, inner, delta, max_iters, mdagm=False):
 
 class MInvCG:
     """mode: 0 host scalars, 1 FP64 scalars in device memory (eager
-    launches), 2 the same with each iteration replayed from a HIP graph
-    (the library's default)."""
+    launches; the library's default), 2 the same with the iterations replayed
+    from HIP graphs."""
 
     def __init__(self, M, max_iters, max_shifts, mode=None):
         self.M = M

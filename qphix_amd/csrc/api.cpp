@@ -86,9 +86,13 @@ struct qphix_solver {
   // operator is not applied to the zero vector
   int x_zero = 0;
   // MInvCG control: 0 host scalars (one host round trip per iteration), 1
-  // FP64 scalars in device memory with eager launches, 2 the same with each
-  // iteration replayed from a HIP graph
-  int ms_mode = 2;
+  // FP64 scalars in device memory with eager launches, 2 the same with the
+  // iterations replayed from HIP graphs (one for each of a round). 1 is the
+  // fastest at every size measured: FP64, modes 0, 1 and 2 in ms, 3 shifts on 4^4,
+  // 12 iterations 0.71, 0.57, 0.96, 40 iterations 2.2, 1.6, 2.2; 12 shifts on
+  // 16^3x32, 12 iterations 2.8, 1.9, 2.1, 40 iterations 9.1, 5.5, 5.9; 12
+  // shifts on 24^3x48, 40 iterations 40.7, 23.6, 24.1
+  int ms_mode = 1;
   // CG and BiCGStab control: 0 host scalars, 1 device scalars (eager
   // launches), 2 device scalars with the iteration replayed from a HIP graph.
   // 1 is the fastest at every size measured (8^4 FP64 CG to 1e-12: 2.37, 1.75
