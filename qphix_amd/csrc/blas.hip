@@ -303,9 +303,14 @@ __device__ inline bool last_block(unsigned *tickets) {
 // t, t + 256, ...) into fin.out and the solver's scalar step. The partials are
 // stored and loaded at agent scope; the wavefront that stored a block's waits
 // for the stores to complete before it counts the block, so the block that
-// reads the full count finds all of them. (An acquire-release increment would
-// order them too, but writes back and invalidates the L2 once per block: 80 us
-// a launch at 2048 blocks.)
+// reads the full count finds all of them. That holds on gfx950, where such
+// stores write through to the device's coherence point before vmcnt counts them
+// done; the language's memory model asks for a release and an acquire. (An
+// acquire-release increment writes back and invalidates the L2 once per block:
+// 80 us a launch at 2048 blocks.)
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "finish_reduction relies on gfx950's write-through agent-scope stores"
+#endif
 template <int NR> __device__ inline void finish_reduction(double *red, const BlasFin &fin) {
   block_reduce_store<NR, true>(red, fin.partials);
   __shared__ double lds[kBlasThreads / 64][NR];
