@@ -24,17 +24,23 @@ constexpr int split_threads(int kind) { return 64 * (8 + split_epi(kind)); }
 // values by the largest of them, and a spin of FP32 is a word and a half
 constexpr bool split_gather(int p, int kind) { return p == P16 || p == PB16 || (p == P32 && kind == KD_FULL); }
 
-
 // Largest number of sites (times right-hand sides) that take this form by
 // rule; from 2^17 sites on, where the hops are tuned, it is a candidate of the
-// tuner instead. The line lies where hop_kernel has about a wavefront per SIMD
-// (65536 sites) and its wider loads per wavefront begin to pay. Measured, A^-1 D
-// psi in us, hop_kernel / this: FP64 2048 sites 10.4 / 5.0, 13824 15.7 / 5.6,
-// 49152 20.6 / 19.6, 65536 23.8 / 24.8; FP32 2048 7.5 / 4.2, 32768 12.4 / 5.3,
-// 96000 18.9 / 15.6, 331776 51.8 / 48.5; FP16 2048 7.1 / 4.7, 32768 8.4 / 5.8,
-// 49152 9.3 / 8.0, 65536 9.7 / 11.3 (Wilson 7.45 / 7.62 at 49152). Full
-// blocks in FP32: 32768 13.4 / 7.3, 49152 14.2 / 12.2, 65536 15.6 / 15.5; in
-// FP16: 32768 9.8 / 5.6.
+// tuner instead. The lines lie where the forms meet: in FP64 and the half
+// precisions, and for full blocks, below a wavefront per SIMD of hop_kernel (65536
+// sites), whose wider loads per wavefront then begin to pay; FP32 keeps its
+// lead to the tuner's range. Measured in us, hop_kernel / this, with the fields
+// in the caches and (in brackets) after 1.2 GB of other traffic, the launch's 3 us
+// included there. A^-1 D psi, FP64: 2048 sites 10.4 / 5.1 (13.7 / 7.7), 13824
+// 16.8 / 5.7 (20.0 / 9.4), 32768 19.2 / 14.1 (22.0 / 16.8), 49152 20.9 / 19.9
+// (24.0 / 22.4), 65536 23.8 / 24.8; FP32: 2048 7.6 / 4.4 (10.6 / 7.0), 32768
+// 12.4 / 5.6 (15.4 / 9.4), 65536 14.1 / 11.8 (17.2 / 14.6), 115200 21.0 / 18.9
+// (24.1 / 21.8), 331776 51.8 / 48.5; FP16: 2048 7.2 / 4.8 (10.1 / 7.4), 32768
+// 8.6 / 6.0 (12.0 / 8.8), 40960 9.3 / 8.4 (12.5 / 11.4), 65536 9.7 / 11.3. The
+// Wilson hop gains least: FP64 49152 17.1 / 16.5 and, on 16x16x24x16, 17.4 / 17.2
+// (19.8 / 19.8, 20.2 / 21.0), FP16 36960 7.3 / 7.6 (10.8 / 10.4). Full blocks:
+// FP64 49152 24.7 / 23.7 (27.8 / 26.5), FP32 49152 14.6 / 12.6 (17.9 / 15.3), 65536
+// 15.6 / 15.5, FP16 32768 9.9 / 6.0 (13.2 / 9.4), 40960 10.5 / 8.3 (13.6 / 12.0).
 constexpr long split_sites(int p, int kind) {
   return p == P64 ? 49152 : p == P32 ? (kind == KD_FULL ? 49152 : (1l << 17) - 1) : 45056;
 }
