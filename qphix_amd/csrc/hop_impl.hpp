@@ -38,15 +38,15 @@ struct HopArgs {
   double ctf, ctb;   // temporal coefficient of the forward hop at t = Nt-1 / backward hop at t = 0
   double tbc_r[4], tbc_i[4];
   int tbc_mask;
+  // the eight terms of a site over wavefronts (hop_split.hpp, natural order):
+  // 1: the tuner's choice, 0: by rule, -1: no, the caller fixed the launch
+  int split;
   double alpha, mu, muinv, rho;
   // traversal: bz = 0 is the natural site order; otherwise the (y, z) cross
   // section is cut into tiles of by rows (by = 0: all of y) by bz planes and
   // each of `slabs` t-slabs is walked tile by tile, t innermost, so consecutive
   // work-groups of one XCD reuse the source spinor slices they share
   int bz, slabs, by;
-  // the eight terms of a site over wavefronts (hop_split.hpp, natural order):
-  // 1: the tuner's choice, 0: by rule, -1: no, the caller fixed the launch
-  int split;
   int dir;  // KD_DIR only
   // multi-RHS: nrhs > 1 applies the operator to psis[r] -> outs[r] (chis[r]);
   // the right-hand side is the fastest index of the work-group order, so the
