@@ -458,7 +458,7 @@ hipError_t mshift_launch(const GeomDesc &g, const MShiftArgs &m, hipStream_t st)
 // ---------------------------------------------------------------------------
 // multishift CG with its scalars in device memory
 //
-// The scalar kernels evaluate the host loop's FP64 expressions in the same
+// The scalar steps evaluate the host loop's FP64 expressions in the same
 // order with contraction off, so each operation rounds as the host's does and
 // the solve is bit-identical to the one with host scalars.
 // ---------------------------------------------------------------------------
@@ -719,7 +719,7 @@ hipError_t ms_set_launch(MsState *st_dev, const MsState &h, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // BiCGStab with its scalars in device memory (invbicgstab.h:150-256)
 //
-// Each kernel evaluates the host loop's expressions in the same order with
+// Each step evaluates the host loop's expressions in the same order with
 // contraction off (the host's flavour sums start from 0, so do these), so
 // the solve is bit-identical to the one with host scalars. A breakdown or the
 // end of the solve freezes the state and sets the skip flag of the vector
